@@ -191,6 +191,45 @@ struct MmParams {
     const void *cb3;        // the codebook's exact bf16 pieces (split_codebook_bf16x3)
 };
 int launch_mm(const MmParams &p, int dtype, hipStream_t st);
+// The block_dim-16 linear for prefill batches (lut_gemm.hip): 16-byte aligned x,
+// K <= 65535; scratch of the calling thread and stream, so not under capture.
+struct LinearGemm {
+    const uint8_t *codes;   // [S][Mp][16]
+    const void *cb_bf16;    // the codebook in bf16, where that is exact, or null
+    const void *cb_half;    // its fp16 pieces, scaled by 2^-ec, or null (split_codebook_half)
+    int ec;
+    const float *scales;    // [M]
+    const float *bias;      // [M] or null
+    // The outliers in groups of four entries of one row, or null: row m's groups
+    // are gptr[m] .. gptr[m + 1] - 1 (one at least), group g's entries ocol and
+    // oval[4 g ..] in column order, the last group filled up with value 0 at
+    // column K; orow[g] = m, with bit 31 set in a row's first group.  Four
+    // readable groups follow the last.
+    const int *gptr, *orow, *ocol;
+    const float *oval;
+    int K, M, Mp;
+};
+bool gemm_pays(const LinearGemm &g, int B, int dtype);   // against lut_mm32_kernel
+int launch_gemm(const LinearGemm &g, const void *x, void *y, int B, int dtype, hipStream_t st);
+// The groups of a CSR whose columns are sorted within rows, on st: gptr [M + 1],
+// the others sized for nnz / 4 + M + 4 groups.
+int launch_outlier_groups(const int *rowp, const int *col, const float *val, int M, int K, int *gptr,
+                          int *ocol, float *oval, int *orow, hipStream_t st);
+constexpr size_t kCbHalf = 2 * 256 * 16, kCbBf16 = 256 * 16;   // values of the two below
+// A 256 x 16 fp32 codebook as fp16 h + l of C * 2^-ec (2^-24 of every value),
+// laid out [piece][half][centroid][8]; false where that is not so: a value is
+// not finite, or a centroid's largest value is below 2^-16 of the codebook's.
+bool split_codebook_half(const float *cb, uint16_t *out, int *ec);
+// The codebook in bf16 laid out [half][centroid][8]; false unless exact.
+bool codebook_bf16(const float *cb, uint16_t *out);
+// Device scratch of the calling thread for work on st, at least n bytes: calls
+// of one thread on one stream are ordered, so they share it; other threads and
+// streams have their own.  At most kScratchStreams streams per thread keep one
+// (the least recently used is freed), and all end with the thread.
+constexpr int kScratchStreams = 4;
+int stream_scratch(hipStream_t st, size_t n, void **out);
+// Whether st can take calls that may allocate: not while it is being captured.
+bool may_allocate(hipStream_t st);
 // One linear handle's forward of B tokens (dtype F32 or BF16) on st.
 int linear_forward(void *h, const void *x, void *y, int B, int dtype, hipStream_t st);
 int linear_forward_fused(void *h, const float *x, float *y, int pro, const float *w, float eps,

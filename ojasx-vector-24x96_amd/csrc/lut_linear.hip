@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <type_traits>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "common.h"
@@ -588,10 +589,16 @@ struct Linear {
     int K = 0, M = 0, D = 0, Kcb = 0, G = 0, S = 0, Mp = 0;
     bool has_bias = false;
     size_t nnz = 0;
+    int ec = 0;                // exponent of cb_half's scale
+    bool half = false, bf16 = false;   // which prefill codebooks follow cb3's pieces
+    // The outliers in groups of four (LinearGemm): made by the first prefill call
+    std::mutex group_lock;
+    bool grouped = false;
+    DevBuf groups;
     DevBuf codes, codes_b, codebook, cb3, scales, bias, rowp, col, col16, val;
     DevBuf lut, xstage, ystage;
     ~Linear() {
-        for (DevBuf *b : {&codes, &codes_b, &codebook, &cb3, &scales, &bias, &rowp, &col, &col16,
+        for (DevBuf *b : {&codes, &codes_b, &codebook, &cb3, &groups, &scales, &bias, &rowp, &col, &col16,
                           &val, &lut, &xstage, &ystage})
             b->release();
     }
@@ -795,6 +802,32 @@ int launch(Linear *L, const void *x, void *y, int B, hipStream_t st) {
 // 17.0 us).
 constexpr int kMmMinBatch = 9;
 
+// The prefill kernel's outlier groups, made on the device by the first call
+// that needs them (one-token callers never pay for them); that call waits for
+// them once, so calls on any stream find them whole.
+int outlier_groups(Linear *L, LinearGemm *g, hipStream_t st) {
+    const int most = (int)(L->nnz / 4) + L->M;   // a row adds at most one partial group
+    const size_t ptr = round_up((size_t)(L->M + 1) * sizeof(int), 64), n = (size_t)most + 4;
+    std::lock_guard<std::mutex> lock(L->group_lock);
+    int rc = L->groups.ensure(ptr + n * 9 * sizeof(int));
+    if (rc) return rc;
+    int *gptr = L->groups.as<int>(), *ocol = gptr + ptr / sizeof(int);
+    float *oval = reinterpret_cast<float *>(ocol + 4 * n);
+    int *orow = reinterpret_cast<int *>(oval + 4 * n);
+    if (!L->grouped) {
+        rc = launch_outlier_groups(L->rowp.as<int>(), L->col.as<int>(), L->val.as<float>(), L->M, L->K,
+                                   gptr, ocol, oval, orow, st);
+        if (rc) return rc;
+        OJX_HIP(hipStreamSynchronize(st));
+        L->grouped = true;
+    }
+    g->gptr = gptr;
+    g->ocol = ocol;
+    g->oval = oval;
+    g->orow = orow;
+    return OJASX_OK;
+}
+
 int forward(Linear *L, const void *x, void *y, int B, int dtype, hipStream_t st) {
     if (B <= 0) return OJASX_OK;
     if (dtype != OJASX_DTYPE_F32 && dtype != OJASX_DTYPE_BF16) {
@@ -807,6 +840,22 @@ int forward(Linear *L, const void *x, void *y, int B, int dtype, hipStream_t st)
     }
     if (L->D == 16 && B >= kMmMinBatch && L->K <= 65535 &&
         (dtype != OJASX_DTYPE_F32 || reinterpret_cast<uintptr_t>(x) % 16 == 0)) {
+        LinearGemm g{};
+        g.codes = L->codes.as<uint8_t>();
+        const uint16_t *pieces = L->cb3.as<uint16_t>() + kCb3Bytes / 2;
+        g.cb_half = L->half ? pieces : nullptr;
+        g.cb_bf16 = L->bf16 ? pieces + kCbHalf : nullptr;
+        g.ec = L->ec;
+        g.scales = L->scales.as<float>();
+        g.bias = L->has_bias ? L->bias.as<float>() : nullptr;
+        g.K = L->K;
+        g.M = L->M;
+        g.Mp = L->Mp;
+        if (reinterpret_cast<uintptr_t>(x) % 16 == 0 && gemm_pays(g, B, dtype) && may_allocate(st)) {
+            int rc = L->nnz ? outlier_groups(L, &g, st) : OJASX_OK;
+            if (!rc) rc = launch_gemm(g, x, y, B, dtype, st);
+            if (rc != OJASX_ERR_OOM) return rc;   // no memory: the kernel below needs none
+        }
         MmParams mp{L->codes.as<uint8_t>(), L->codebook.as<float>(), L->scales.as<float>(),
                     L->has_bias ? L->bias.as<float>() : nullptr,
                     L->nnz ? L->rowp.as<int>() : nullptr, L->col.as<int>(), L->val.as<float>(),
@@ -1000,9 +1049,12 @@ OJASX_API OjasxLinearHandle ojasx_create_linear(int in_features, int out_feature
     }
     if (!rc) rc = upload(L->codebook, cb.data(), cb.size() * sizeof(float));
     if (!rc && L->D == 16) {   // the grouped kernel's MFMA operand
-        std::vector<uint16_t> cb3(kCb3Bytes / 2);
+        // the three pieces, then the prefill kernel's operands: fp16 halves, bf16
+        std::vector<uint16_t> cb3(kCb3Bytes / 2 + kCbHalf + kCbBf16);
         split_codebook_bf16x3(cb.data(), cb3.data());
-        rc = upload(L->cb3, cb3.data(), kCb3Bytes);
+        L->half = split_codebook_half(cb.data(), cb3.data() + kCb3Bytes / 2, &L->ec);
+        L->bf16 = codebook_bf16(cb.data(), cb3.data() + kCb3Bytes / 2 + kCbHalf);
+        rc = upload(L->cb3, cb3.data(), cb3.size() * 2);
     }
     if (!rc) rc = upload(L->scales, sc.data(), sc.size() * sizeof(float));
     if (!rc && bias_data) {
@@ -1075,6 +1127,7 @@ OJASX_API int ojasx_set_linear_outliers(OjasxLinearHandle handle, int nnz, const
     }
     if (rc) return rc;
     L->nnz = (size_t)nnz;
+    L->grouped = false;
     return OJASX_OK;
 }
 
