@@ -327,30 +327,6 @@ constexpr int kM32NT = 512;      // threads: 8 waves
 template <typename T> constexpr bool kM32RowPairs = std::is_same<T, float>::value;
 }  // namespace
 
-// Exact three-way bf16 split of 8 fp32 values by truncation: v = p0 + p1 + p2,
-// p0 = v with its low 16 bits cleared, p1 the same of v - p0, p2 = v - p0 - p1
-// (the remainders are exact in fp32; p2 has at most 8 significant bits, a
-// bf16 value).  |p1| < 2^-7 |v|, |p2| < 2^-15 |v|.  About five operations per
-// value (1.5 of them packing).
-__device__ __forceinline__ void split3_trunc(const float (&v)[8], bf16x8_t (&p)[3]) {
-    uint32_t w[3][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t ua = __float_as_uint(v[2 * i]), ub = __float_as_uint(v[2 * i + 1]);
-        const float ra = v[2 * i] - __uint_as_float(ua & 0xffff0000u);
-        const float rb = v[2 * i + 1] - __uint_as_float(ub & 0xffff0000u);
-        const uint32_t ura = __float_as_uint(ra), urb = __float_as_uint(rb);
-        const float sa = ra - __uint_as_float(ura & 0xffff0000u);
-        const float sb = rb - __uint_as_float(urb & 0xffff0000u);
-        // high halves of (a, b) into one word, element 2i in its low half
-        w[0][i] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-        w[1][i] = __builtin_amdgcn_perm(urb, ura, 0x07060302u);
-        w[2][i] = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) __builtin_memcpy(&p[k], w[k], sizeof(bf16x8_t));
-}
-
 template <typename T, int RT, int TT>
 __global__ __launch_bounds__(kM32NT) void lut_mm32_kernel(MmParams p) {
     constexpr int KP = kM32NT / 64;               // input parts, one wave each
