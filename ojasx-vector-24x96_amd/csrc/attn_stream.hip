@@ -12,6 +12,7 @@
 // contiguous in the state.
 //
 // One update call folds a list of tiles, in order, into the state:
+//  * many query rows: attn_rows_kernel below, on fp64 MFMA; otherwise
 //  * attn_tile_kernel -- workgroup = (chunk of up to 256 tokens of one tile,
 //    batch x kv head, block of RB rows of that kv head's query rows).
 //    Scores: thread t owns token t, s_r = (<q_r, k_t> * kscale_t) * scale in
@@ -323,6 +324,266 @@ __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
     }
 }
 
+// attn_rows_kernel: the same fold on v_mfma_f64_16x16x4f64 for many query rows
+// (prefill): workgroup = 64 query rows of one kv head (16 per wave) over a run
+// of the work items, 32 tokens at a time.
+//  * K and V of a step are converted to fp64 once, into LDS (the next step's raw
+//    16-byte pieces are loaded meanwhile); a wave's q stays in registers.
+//  * S^T = K Q^T: tokens are the MFMA's rows, query rows its columns, so lane l
+//    holds query l % 16 and register r of token tile tt token 16 tt + 4 r + l/16:
+//    just what the B operand of O^T = V^T P^T takes in step (tt, r).  The
+//    probabilities never leave their lane; the row maximum crosses lanes twice
+//    per step.
+//  * The online update is the reference's (:129-163) per 32 tokens; row bounds
+//    past R, tokens past the item and causally hidden ones score -inf, and a
+//    step whose first token no row may see ends the run.
+// With one run the accumulators start from the state and go back to it; with
+// several (too few row blocks for the chip) each run leaves partials for
+// attn_merge_kernel.
+// LDS rows are padded so that the K reads (16 tokens x 4 dims) and V reads (4
+// tokens x 16 dims) of a half-wave meet all 32 8-byte banks once.
+// What bounds it: the fp64 matrix rate (74 TFLOP/s measured on this card, 59
+// for fp64 FMAs on the VALU), the longest row block's tokens where the mask
+// leaves others fewer, and what does not overlap (copies without a part run 42 us
+// faster without the exponentials, 49 without the conversion of K and V).  The
+// kernel above runs the dots on the VALU with q through scalar loads, again for
+// every 8 rows: 512 causal queries of 32 heads over 2048 tokens (8 kv heads, dim
+// 128, bf16), four calls of 146 us and their merges of 14 against one of 362.
+namespace {
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+constexpr int kRNT = 512;            // threads
+constexpr int kRT = 32;              // tokens per step, 16 per wave
+constexpr int kRRows = 64;           // query rows per workgroup
+constexpr int pad_to(int d, int mod) { return d + ((mod - d % 32) + 32) % 32; }
+}  // namespace
+
+template <int KT, int D>
+__global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(KT == KV_F64 && D == 128 ? 1 : 2)))
+void attn_rows_kernel(AttnParams p, double *state, int n_work) {
+    typedef typename Elem<KT>::T T;
+    constexpr bool kI8 = KT == KV_INT8;
+    constexpr int PK = pad_to(D, 2), PV = pad_to(D, 16);
+    constexpr int kE = 16 / (int)sizeof(T);          // elements per 16-byte piece
+    constexpr int NP = kRT * D / kE;                 // pieces of a step's K (and V)
+    constexpr int NU = (NP + kRNT - 1) / kRNT;
+    typedef unsigned int v4u __attribute__((ext_vector_type(4), aligned(4)));
+    extern __shared__ __align__(16) unsigned char asm_[];
+    // per buffer: K [32][PK], V [32][PV], int8: the scales of K and V [2][32]
+    constexpr int kBuf = kRT * (PK + PV + 2);
+    double *lds = reinterpret_cast<double *>(asm_);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int c = lane & 15, g = lane >> 4, wr = w & 3, wt = w >> 2;   // rows 16 wr .., tokens 16 wt ..
+    const int bh = blockIdx.y, b = bh / p.Hkv, h = bh - b * p.Hkv;
+    const int nz = gridDim.z, z = blockIdx.z;
+    const int w0 = (int)((long long)n_work * z / nz), w1 = (int)((long long)n_work * (z + 1) / nz);
+    const int r0 = blockIdx.x * kRRows, row = r0 + 16 * wr + c;
+    const bool rok = row < p.R;
+    double *st = state + ((size_t)bh * p.R + min(row, p.R - 1)) * (2 * D + 2);
+    const long long qpos = p.qsp + min(row, p.R - 1) % p.Sq;
+    // the last position any of the block's rows may see
+    const int rl = min(r0 + kRRows, p.R) - 1;
+    const long long top = p.causal ? p.qsp + (r0 / p.Sq == rl / p.Sq ? rl % p.Sq : p.Sq - 1) : 0x7fffffffffffffffLL;
+
+    uint4 kr[NU], vr[NU];
+    double scr = 0.0;
+    auto load = [&](const AttnWork &wk, const AttnTile &tl, int t0) __attribute__((always_inline)) {
+        const T *kb = static_cast<const T *>(tl.k) + b * tl.sb + h * tl.sh;
+        const T *vb = static_cast<const T *>(tl.v) + b * tl.sb + h * tl.sh;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int i = min(tid + u * kRNT, NP - 1), t = i / (D / kE), e = i % (D / kE) * kE;
+            const long long at = (long long)(wk.t0 + min(t0 + t, wk.n - 1)) * tl.st + e;
+            kr[u] = gld(reinterpret_cast<const uint4 *>(kb + at));
+            const v4u v = gld(reinterpret_cast<const v4u *>(vb + at));   // 4-element aligned
+            vr[u] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+        if constexpr (kI8)
+            if (tid < 2 * kRT) {
+                const __half *sp = (tid < kRT ? tl.ks : tl.vs) + b * tl.ssb + h * tl.ssh;
+                scr = (double)__half2float(__ushort_as_half(gld(reinterpret_cast<const unsigned short *>(
+                    sp + (wk.t0 + min(t0 + (tid & (kRT - 1)), wk.n - 1)) * tl.sst))));
+            }
+    };
+    // A piece's doubles go out 16 bytes at a time, in an order turned by the lane
+    // so that 16 lanes of a write meet all 16 four-bank groups.
+    auto put = [&](double *dst, const uint4 &raw) __attribute__((always_inline)) {
+        typedef double d2 __attribute__((ext_vector_type(2)));
+        if constexpr (sizeof(T) == 8) {
+            *reinterpret_cast<uint4 *>(dst) = raw;
+        } else if constexpr (sizeof(T) == 4) {
+            const bool sw = lane & 8;
+            const uint32_t a0 = sw ? raw.z : raw.x, a1 = sw ? raw.w : raw.y;
+            const uint32_t b0 = sw ? raw.x : raw.z, b1 = sw ? raw.y : raw.w;
+            *reinterpret_cast<d2 *>(dst + (sw ? 2 : 0)) = d2{(double)__uint_as_float(a0), (double)__uint_as_float(a1)};
+            *reinterpret_cast<d2 *>(dst + (sw ? 0 : 2)) = d2{(double)__uint_as_float(b0), (double)__uint_as_float(b1)};
+        } else {
+            const int rot = (kI8 ? lane >> 1 : lane >> 2) & 3;
+            uint32_t v[4] = {raw.x, raw.y, raw.z, raw.w}, t[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[j] = rot & 1 ? v[(j + 1) & 3] : v[j];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = rot & 2 ? t[(j + 2) & 3] : t[j];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                double *at = dst + ((j + rot) & 3) * (kE / 4);
+                T e[kE / 4];
+                __builtin_memcpy(e, &v[j], 4);
+                if constexpr (kI8) {
+                    const bool sw = lane & 8;
+                    *reinterpret_cast<d2 *>(at + (sw ? 2 : 0)) = d2{to_d(sw ? e[2] : e[0]), to_d(sw ? e[3] : e[1])};
+                    *reinterpret_cast<d2 *>(at + (sw ? 0 : 2)) = d2{to_d(sw ? e[0] : e[2]), to_d(sw ? e[1] : e[3])};
+                } else {
+                    *reinterpret_cast<d2 *>(at) = d2{to_d(e[0]), to_d(e[1])};
+                }
+            }
+        }
+    };
+    auto store = [&](double *buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int i = tid + u * kRNT;
+            if (NP % kRNT && i >= NP) break;
+            const int t = i / (D / kE), e = i % (D / kE) * kE;
+            put(buf + t * PK + e, kr[u]);
+            put(buf + kRT * PK + t * PV + e, vr[u]);
+        }
+        if constexpr (kI8)
+            if (tid < 2 * kRT) buf[kRT * (PK + PV) + tid] = scr;
+    };
+
+    double q[D / 4];
+#pragma unroll
+    for (int k = 0; k < D / 4; ++k) q[k] = st[4 * k + g];
+    f64x4_t o[D / 16];
+    double m = -INFINITY, l = 0.0;
+#pragma unroll
+    for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[d][r] = nz == 1 && wt == 0 ? st[D + 16 * d + 4 * r + g] : 0.0;
+    if (nz == 1 && wt == 0) {
+        m = st[2 * D];
+        l = g == 0 ? st[2 * D + 1] : 0.0;
+    }
+
+    if (w0 < w1) {
+        // the step being loaded: item wi, its tokens t0 ..
+        int wi = w0, t0 = 0;
+        AttnWork wk = p.work[wi];
+        AttnTile tl = p.tiles[wk.tile];
+        int n = min(kRT, wk.n);                      // of the step being computed
+        long long pos = wk.pos;
+        auto next = [&]() __attribute__((always_inline)) {
+            t0 += kRT;
+            if (t0 >= wk.n) {
+                t0 = 0;
+                if (++wi < w1) {
+                    wk = p.work[wi];
+                    tl = p.tiles[wk.tile];
+                }
+            }
+            return wi < w1 && wk.pos + t0 <= top;
+        };
+        bool cur = pos <= top, more = false;
+        if (cur) {
+            load(wk, tl, 0);
+            store(lds);
+            more = next();
+            if (more) load(wk, tl, t0);
+        }
+        __syncthreads();
+        for (int par = 0; cur; par ^= 1) {
+            const double *buf = lds + par * kBuf;
+            int n1 = 0;
+            long long pos1 = 0;
+            bool more1 = false;
+            if (more) {
+                store(lds + (par ^ 1) * kBuf);
+                n1 = min(kRT, wk.n - t0);
+                pos1 = wk.pos + t0;
+                more1 = next();
+                if (more1) load(wk, tl, t0);
+            }
+            f64x4_t s = {};
+            const double *ka = buf + (16 * wt + c) * PK + g;
+#pragma unroll
+            for (int k = 0; k < D / 4; ++k)
+                s = __builtin_amdgcn_mfma_f64_16x16x4f64(ka[4 * k], q[k], s, 0, 0, 0);
+            double mx = -INFINITY, vs[4];
+            const double *sc = buf + kRT * (PK + PV);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int tk = 16 * wt + 4 * r + g;
+                const double ksc = kI8 ? sc[tk] : 1.0;
+                vs[r] = kI8 ? sc[kRT + tk] : 1.0;
+                const bool hide = tk >= n || (p.causal && pos + tk > qpos);
+                s[r] = hide ? -INFINITY : (s[r] * ksc) * p.scale;
+                mx = fmax(mx, s[r]);
+            }
+            mx = fmax(mx, __shfl_xor(mx, 16, 64));
+            mx = fmax(mx, __shfl_xor(mx, 32, 64));
+            const double mn = fmax(m, mx);
+            const double safe = isinf(mn) ? 0.0 : mn;
+            if (__any(mn != m || m == INFINITY)) {
+                const double f = isinf(m) ? 0.0 : exp(m - safe);
+                l *= f;
+#pragma unroll
+                for (int d = 0; d < D / 16; ++d) o[d] *= f;
+                m = mn;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double pr = isinf(s[r]) ? 0.0 : exp(s[r] - safe);
+                l += pr;
+                s[r] = pr * vs[r];
+            }
+            const double *va = buf + kRT * PK + (16 * wt + g) * PV + c;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int d = 0; d < D / 16; ++d)
+                    o[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[4 * r * PV + 16 * d], s[r], o[d], 0, 0, 0);
+            __syncthreads();   // the next step is staged, this one's buffer free
+            n = n1;
+            pos = pos1;
+            cur = more;
+            more = more1;
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    // the second half's sums into the first's (the buffers are free)
+    double *mg = reinterpret_cast<double *>(asm_) + (size_t)wr * 64 * (D / 4 + 2) + lane;
+    if (wt == 1) {
+#pragma unroll
+        for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mg[64 * (4 * d + r)] = o[d][r];
+        mg[64 * (D / 4)] = m;
+        mg[64 * (D / 4 + 1)] = l;
+    }
+    __syncthreads();
+    if (wt == 1 || !rok) return;
+    {
+        const double m1 = mg[64 * (D / 4)], mn = fmax(m, m1), safe = isinf(mn) ? 0.0 : mn;
+        const double f0 = isinf(m) ? 0.0 : exp(m - safe), f1 = isinf(m1) ? 0.0 : exp(m1 - safe);
+        l = f0 * l + f1 * mg[64 * (D / 4 + 1)];
+        m = mn;
+#pragma unroll
+        for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[d][r] = f0 * o[d][r] + f1 * mg[64 * (4 * d + r)];
+    }
+    double *dst = nz == 1 ? st + D : p.part + ((size_t)z * p.rows + (size_t)bh * p.R + row) * (D + 2);
+#pragma unroll
+    for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dst[16 * d + 4 * r + g] = o[d][r];
+    if (g == 0) {
+        dst[D] = m;
+        dst[D + 1] = l;
+    }
+}
+
 // State row `blockIdx.x` <- the state merged with the n partials: the maximum
 // over all, then thread (4 dims dq, phase ph) sums f_i * acc_i over partials
 // i = ph, ph + PH, ... (f_i = exp(m_i - m), 0 for m_i = -inf), and the phases
@@ -484,6 +745,36 @@ int launch_tiles(const AttnParams &p, int n_work, int B, int RB, hipStream_t st)
     OJX_HIP(hipGetLastError());
     return OJASX_OK;
 }
+
+template <int KT, int D>
+int launch_rows_d(const AttnParams &p, double *state, int n_work, dim3 grid, hipStream_t st) {
+    constexpr size_t lds = (size_t)2 * kRT * (pad_to(D, 2) + pad_to(D, 16) + 2) * sizeof(double);
+    static size_t granted = 0;
+    int rc = ensure_dyn_lds(reinterpret_cast<const void *>(&attn_rows_kernel<KT, D>), lds, &granted);
+    if (rc) return rc;
+    OJX_LAUNCH((attn_rows_kernel<KT, D>), grid, dim3(kRNT), lds, st, p, state, n_work);
+    OJX_HIP(hipGetLastError());
+    return OJASX_OK;
+}
+
+template <int KT>
+int launch_rows(const AttnParams &p, double *state, int n_work, dim3 grid, hipStream_t st) {
+    switch (p.D) {
+        case 64: return launch_rows_d<KT, 64>(p, state, n_work, grid, st);
+        case 80: return launch_rows_d<KT, 80>(p, state, n_work, grid, st);
+        default: return launch_rows_d<KT, 128>(p, state, n_work, grid, st);
+    }
+}
+
+// attn_rows_kernel from 64 rows per kv head (head dims 64, 80, 128) and 128
+// blocks of 64 rows x 256 tokens.  A block takes it 54 us whatever else runs, up
+// to 256 at once; attn_tile_kernel takes about 20 us and 0.32 us per block (64
+// rows of 8 kv heads over 2048 tokens, 64 blocks: 54 against 38 us; 512 rows,
+// 512 blocks: 106 against 180).
+bool rows_kernel(int R, int D, long groups, long tokens) {
+    return R >= kRRows && (D == 64 || D == 80 || D == 128) &&
+           tokens / kACH * ((R + kRRows - 1) / kRRows) * groups >= 128;
+}
 }  // namespace
 
 }  // namespace ojx
@@ -608,8 +899,6 @@ OJASX_API int ojasx_attention_stream_update_device(double *state, int batch, int
     const size_t per_work = (size_t)rows * (D + 2) * sizeof(double);
     const int n_work = (int)wl.size();
     const int per_round = (int)std::max<size_t>(1, std::min<size_t>(n_work, kPartCap / per_work));
-    rc = sg.part.ensure(per_work * per_round);
-    if (rc) return rc;
     int RB = 8;
     while (RB > 1 && RB / 2 >= R) RB /= 2;
     if ((R + RB - 1) / RB > 65535) {
@@ -619,7 +908,6 @@ OJASX_API int ojasx_attention_stream_update_device(double *state, int batch, int
     AttnParams p{};
     p.tiles = static_cast<const AttnTile *>(staged);
     p.state = state;
-    p.part = sg.part.as<double>();
     p.qsp = query_start_pos;
     p.scale = scale;
     p.Hkv = num_kv_heads;
@@ -628,6 +916,36 @@ OJASX_API int ojasx_attention_stream_update_device(double *state, int batch, int
     p.D = D;
     p.rows = rows;
     p.causal = causal != 0;
+    if (rows_kernel(R, D, (long)batch * num_kv_heads, (long)(pos - kv_offset))) {
+        // a workgroup per CU of 256; runs beyond the row blocks leave partials
+        const long blocks = (long)((R + kRRows - 1) / kRRows) * batch * num_kv_heads;
+        long nz = std::min<long>({256 / blocks, (long)n_work, 65535L, (long)(kPartCap / per_work)});
+        if (nz < 1) nz = 1;
+        if (nz > 1) {
+            rc = sg.part.ensure(per_work * nz);
+            if (rc) return rc;
+        }
+        p.part = sg.part.as<double>();
+        p.work = reinterpret_cast<const AttnWork *>(static_cast<unsigned char *>(staged) + tile_bytes);
+        const dim3 grid((R + kRRows - 1) / kRRows, batch * num_kv_heads, (unsigned)nz);
+        switch (kv_dtype) {
+            case KV_F32: rc = launch_rows<KV_F32>(p, state, n_work, grid, st); break;
+            case KV_BF16: rc = launch_rows<KV_BF16>(p, state, n_work, grid, st); break;
+            case KV_F16: rc = launch_rows<KV_F16>(p, state, n_work, grid, st); break;
+            case KV_F64: rc = launch_rows<KV_F64>(p, state, n_work, grid, st); break;
+            default: rc = launch_rows<KV_INT8>(p, state, n_work, grid, st); break;
+        }
+        if (rc) return rc;
+        if (nz > 1) {
+            OJX_LAUNCH(attn_merge_kernel, dim3(rows), dim3(kANT), 0, st, state, (const double *)p.part,
+                       (int)nz, rows, D);
+            OJX_HIP(hipGetLastError());
+        }
+        return sg.ring.launched(st);
+    }
+    rc = sg.part.ensure(per_work * per_round);
+    if (rc) return rc;
+    p.part = sg.part.as<double>();
     const AttnWork *work_dev = reinterpret_cast<const AttnWork *>(static_cast<unsigned char *>(staged) + tile_bytes);
     for (int w0 = 0; w0 < n_work; w0 += per_round) {
         const int n = std::min(per_round, n_work - w0);

@@ -237,6 +237,8 @@ class OnlineSoftmaxBlockAttention:
     1/sqrt(head_dim) follow the reference; the arithmetic runs on the GPU
     (scores and state in fp64, tiles read in their own type)."""
 
+    _STATE_BYTES = 256 << 20         # fp64 state of one pass of ``forward``
+
     def __init__(self, num_heads: int, num_kv_heads: Optional[int] = None, head_dim: int = 64,
                  *, q_block_size: int = 128, kv_block_size: int = 256,
                  causal: bool = True) -> None:
@@ -389,8 +391,8 @@ class OnlineSoftmaxBlockAttention:
     def forward(self, query, key, value, *, query_start_pos: int = 0):
         """Tiled exact attention of ``query`` over ``key`` / ``value``
         [B, H_kv, S_k, D] (long_context.py:178-209): query blocks of
-        q_block_size, each over the kv blocks of kv_block_size its causal
-        horizon reaches, all of a query block's kv blocks in one update."""
+        q_block_size over the kv blocks of kv_block_size their causal horizon
+        reaches, many query blocks and all their kv blocks in one update."""
         torch = _torch()
         self._check_query(query)
         B, H_q, S_q, D = query.shape
@@ -400,9 +402,13 @@ class OnlineSoftmaxBlockAttention:
         self._check_block(value, B, "value")
         key, value, qp = self._pad_d(key), self._pad_d(value), self._pad_d(query)
         S_k = key.shape[2]
+        # whole query blocks per pass: as many as keep the fp64 state (query,
+        # sums, maximum and weight of every row) within _STATE_BYTES
+        per_query = 8 * B * H_q * (2 * self._dpad + 2)
+        step = max(1, self._STATE_BYTES // (per_query * self.q_block_size)) * self.q_block_size
         outs = []
-        for q_start in range(0, S_q, self.q_block_size):
-            q_stop = min(q_start + self.q_block_size, S_q)
+        for q_start in range(0, S_q, step):
+            q_stop = min(q_start + step, S_q)
             q_chunk = qp[:, :, q_start:q_stop, :]
             eff_k = min(S_k, query_start_pos + q_stop) if self.causal else S_k
             state = self._init(q_chunk)
@@ -415,7 +421,7 @@ class OnlineSoftmaxBlockAttention:
             if tiles:
                 self._update(state, q_chunk, tiles, tag, query_start_pos + q_start, 0)
             outs.append(self._finalize(state, q_chunk))
-        out = torch.cat(outs, dim=2)
+        out = outs[0] if len(outs) == 1 else torch.cat(outs, dim=2)
         return out if qp is query else out[..., :D].contiguous()
 
     __call__ = forward
