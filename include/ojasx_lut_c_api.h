@@ -220,6 +220,16 @@ OJASX_API int ojasx_kv_encode_append_device(const float *k, const float *v, int 
                                             int num_pages, uint8_t *k_codes, float *k_scales,
                                             uint8_t *v_codes, float *v_scales, void *stream);
 
+/* ojasx_kv_encode_append_device with slot_mapping [num_tokens] in host memory,
+ * read during the call, for at most 64 tokens: the slots travel with the launch
+ * (a captured launch keeps them). */
+OJASX_API int ojasx_kv_encode_append_host_slots(const float *k, const float *v, int num_tokens,
+                                                int num_kv_heads, int head_dim, int block_dim,
+                                                const float *k_codebook, const float *v_codebook,
+                                                const int *slot_mapping, int page_size,
+                                                int num_pages, uint8_t *k_codes, float *k_scales,
+                                                uint8_t *v_codes, float *v_scales, void *stream);
+
 /* PagedCompressedKVCache._quantize_int8 (ojasx_24x96/long_context.py:234-240)
  * on device: rows of dim elements of x (dtype F32, BF16, F16 or F64), row r of
  * group g at x + g*x_group_stride + r*dim (elements), int8 codes to

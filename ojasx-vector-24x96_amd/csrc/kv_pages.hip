@@ -136,13 +136,19 @@ __global__ __launch_bounds__(kNT) void dequantize_int8_kernel(const int8_t *__re
     store_act(out, i, (float)q[g * q_gs + e] * s);
 }
 
+// Tokens whose slots fit the kernel arguments: a decode step's slot then needs no
+// copy to the device of its own (a synchronising 4-byte copy took longer than
+// the 5 us kernel).
+constexpr int kInlineSlots = 64;
+
 struct EncodeParams {
     const float *k, *v;         // [n][Hkv][hd]
     const float *kcb, *vcb;     // [Hkv][256][D], or both NULL
-    const int *slots;           // [n]
+    const int *slots;           // [n], or NULL: inl
     uint8_t *kc, *vc;           // [pages][Hkv][P][G]
     float *ks, *vs;             // [pages][Hkv][P]
     int Hkv, hd, D, G, P, num_pages;
+    int inl[kInlineSlots];
 };
 
 // Workgroup (token i, kv head h, z): z = 0 encodes the token's K row, z = 1
@@ -158,12 +164,63 @@ __global__ __launch_bounds__(kNT) void kv_encode_append_kernel(EncodeParams p) {
         cb += (size_t)h * 256 * p.D;
         enc_load_centroid<DT>(cb, creg);
     }
-    const int slot = p.slots[i];
+    const int slot = p.slots ? p.slots[i] : p.inl[i];
     if (slot < 0 || slot / p.P >= p.num_pages) return;   // skipped slot; workgroup-uniform
     const int page = slot / p.P;
     const size_t row = ((size_t)page * p.Hkv + h) * p.P + (slot - page * p.P);
     encode_row<DT>((kv ? p.v : p.k) + ((size_t)i * p.Hkv + h) * p.hd, cb, creg, p.hd, p.D, p.G,
                    (kv ? p.vc : p.kc) + row * p.G, (kv ? p.vs : p.ks) + row, xs);
+}
+
+int kv_encode_append(const float *k, const float *v, int num_tokens,
+                                            int num_kv_heads, int head_dim, int block_dim,
+                                            const float *k_codebook, const float *v_codebook,
+                                            const int *slot_mapping, bool host_slots, int page_size,
+                                            int num_pages, uint8_t *k_codes, float *k_scales, uint8_t *v_codes,
+                                            float *v_scales, void *stream) {
+    if (!k || !v || !slot_mapping || !k_codes || !k_scales || !v_codes || !v_scales)
+        return OJASX_ERR_NULL;
+    if ((k_codebook == nullptr) != (v_codebook == nullptr)) {
+        set_error("k_codebook and v_codebook must both be given or both be NULL");
+        return OJASX_ERR_NULL;
+    }
+    if (num_tokens < 0 || num_kv_heads <= 0 || num_kv_heads > 65535 || head_dim <= 0 ||
+        block_dim <= 0 || head_dim % block_dim || head_dim / block_dim > kMaxEncGroups ||
+        head_dim > 16384 || page_size <= 0 || num_pages <= 0) {
+        set_error("invalid KV append shape (head_dim %d, block_dim %d: at most %d groups)",
+                  head_dim, block_dim, kMaxEncGroups);
+        return OJASX_ERR_INVALID;
+    }
+    if (num_tokens == 0) return OJASX_OK;
+    if (host_slots && num_tokens > kInlineSlots) {
+        set_error("at most %d tokens per call with host slots (got %d)", kInlineSlots, num_tokens);
+        return OJASX_ERR_INVALID;
+    }
+    EncodeParams p{k, v, k_codebook, v_codebook, host_slots ? nullptr : slot_mapping, k_codes, v_codes, k_scales,
+                   v_scales, num_kv_heads, head_dim, block_dim, head_dim / block_dim, page_size,
+                   num_pages, {}};
+    if (host_slots) memcpy(p.inl, slot_mapping, (size_t)num_tokens * sizeof(int));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const size_t lds = (size_t)head_dim * sizeof(float);
+    const dim3 grid(num_tokens, num_kv_heads, 2);   // z: K, then V
+    const bool reg16 = block_dim == 16 && k_codebook &&
+                       (reinterpret_cast<uintptr_t>(k_codebook) & 15) == 0 &&
+                       (reinterpret_cast<uintptr_t>(v_codebook) & 15) == 0;
+    if (reg16) {
+        static size_t granted = 0;
+        int rc = ensure_dyn_lds(reinterpret_cast<const void *>(&kv_encode_append_kernel<16>), lds,
+                                &granted);
+        if (rc) return rc;
+        OJX_LAUNCH(kv_encode_append_kernel<16>, grid, dim3(kNT), lds, st, p);
+    } else {
+        static size_t granted = 0;
+        int rc = ensure_dyn_lds(reinterpret_cast<const void *>(&kv_encode_append_kernel<0>), lds,
+                                &granted);
+        if (rc) return rc;
+        OJX_LAUNCH(kv_encode_append_kernel<0>, grid, dim3(kNT), lds, st, p);
+    }
+    OJX_HIP(hipGetLastError());
+    return OJASX_OK;
 }
 
 }  // namespace ojx
@@ -253,45 +310,20 @@ OJASX_API int ojasx_kv_encode_append_device(const float *k, const float *v, int 
                                             const int *slot_mapping, int page_size,
                                             int num_pages, uint8_t *k_codes, float *k_scales, uint8_t *v_codes,
                                             float *v_scales, void *stream) {
-    using namespace ojx;
-    if (!k || !v || !slot_mapping || !k_codes || !k_scales || !v_codes || !v_scales)
-        return OJASX_ERR_NULL;
-    if ((k_codebook == nullptr) != (v_codebook == nullptr)) {
-        set_error("k_codebook and v_codebook must both be given or both be NULL");
-        return OJASX_ERR_NULL;
-    }
-    if (num_tokens < 0 || num_kv_heads <= 0 || num_kv_heads > 65535 || head_dim <= 0 ||
-        block_dim <= 0 || head_dim % block_dim || head_dim / block_dim > kMaxEncGroups ||
-        head_dim > 16384 || page_size <= 0 || num_pages <= 0) {
-        set_error("invalid KV append shape (head_dim %d, block_dim %d: at most %d groups)",
-                  head_dim, block_dim, kMaxEncGroups);
-        return OJASX_ERR_INVALID;
-    }
-    if (num_tokens == 0) return OJASX_OK;
-    EncodeParams p{k, v, k_codebook, v_codebook, slot_mapping, k_codes, v_codes, k_scales,
-                   v_scales, num_kv_heads, head_dim, block_dim, head_dim / block_dim, page_size,
-                   num_pages};
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const size_t lds = (size_t)head_dim * sizeof(float);
-    const dim3 grid(num_tokens, num_kv_heads, 2);   // z: K, then V
-    const bool reg16 = block_dim == 16 && k_codebook &&
-                       (reinterpret_cast<uintptr_t>(k_codebook) & 15) == 0 &&
-                       (reinterpret_cast<uintptr_t>(v_codebook) & 15) == 0;
-    if (reg16) {
-        static size_t granted = 0;
-        int rc = ensure_dyn_lds(reinterpret_cast<const void *>(&kv_encode_append_kernel<16>), lds,
-                                &granted);
-        if (rc) return rc;
-        OJX_LAUNCH(kv_encode_append_kernel<16>, grid, dim3(kNT), lds, st, p);
-    } else {
-        static size_t granted = 0;
-        int rc = ensure_dyn_lds(reinterpret_cast<const void *>(&kv_encode_append_kernel<0>), lds,
-                                &granted);
-        if (rc) return rc;
-        OJX_LAUNCH(kv_encode_append_kernel<0>, grid, dim3(kNT), lds, st, p);
-    }
-    OJX_HIP(hipGetLastError());
-    return OJASX_OK;
+    return ojx::kv_encode_append(k, v, num_tokens, num_kv_heads, head_dim, block_dim, k_codebook, v_codebook,
+                                 slot_mapping, false, page_size, num_pages, k_codes, k_scales, v_codes,
+                                 v_scales, stream);
+}
+
+OJASX_API int ojasx_kv_encode_append_host_slots(const float *k, const float *v, int num_tokens,
+                                            int num_kv_heads, int head_dim, int block_dim,
+                                            const float *k_codebook, const float *v_codebook,
+                                            const int *slot_mapping, int page_size,
+                                            int num_pages, uint8_t *k_codes, float *k_scales, uint8_t *v_codes,
+                                            float *v_scales, void *stream) {
+    return ojx::kv_encode_append(k, v, num_tokens, num_kv_heads, head_dim, block_dim, k_codebook, v_codebook,
+                                 slot_mapping, true, page_size, num_pages, k_codes, k_scales, v_codes,
+                                 v_scales, stream);
 }
 
 }  // extern "C"

@@ -563,16 +563,20 @@ class PagedCodeKVCache:
         self.total_tokens_seen += n
         if n == 0:
             return
-        slots = torch.from_numpy(self.table.plan(n)).to(self.device)
+        slots = self.table.plan(n)
+        if n <= 64:                      # the slots travel with the launch
+            fn, at = _lib.lib().ojasx_kv_encode_append_host_slots, slots.ctypes.data
+        else:
+            slots = torch.from_numpy(slots).to(self.device)
+            fn, at = _lib.lib().ojasx_kv_encode_append_device, slots.data_ptr()
         k = k.to(torch.float32).contiguous()
         v = v.to(torch.float32).contiguous()
         cbk = None if self.scalar_codes else _vp(self.k_codebook)
         cbv = None if self.scalar_codes else _vp(self.v_codebook)
-        rc = _lib.lib().ojasx_kv_encode_append_device(
-            _vp(k), _vp(v), n, self.num_kv_heads, self.head_dim, self.block_dim, cbk, cbv,
-            _vp(slots), self.page_size, self.max_resident_pages, _vp(self.k_codes),
-            _vp(self.k_scales), _vp(self.v_codes), _vp(self.v_scales), _stream())
-        _lib.check(rc, "ojasx_kv_encode_append_device")
+        rc = fn(_vp(k), _vp(v), n, self.num_kv_heads, self.head_dim, self.block_dim, cbk, cbv,
+                at, self.page_size, self.max_resident_pages, _vp(self.k_codes),
+                _vp(self.k_scales), _vp(self.v_codes), _vp(self.v_scales), _stream())
+        _lib.check(rc, "ojasx_kv_encode_append")
 
     @property
     def seq_len(self) -> int:
@@ -601,9 +605,10 @@ class PagedCodeKVCache:
         if q.dim() != 2 or q.shape[1] != self.head_dim or Hq % self.num_kv_heads:
             raise ValueError("q must be [num_q_heads, head_dim], num_q_heads a multiple of "
                              "num_kv_heads")
-        if out is None:
-            out = torch.zeros(Hq, self.head_dim, dtype=torch.float32, device=q.device)
         T = self.seq_len
+        if out is None:                  # written whole unless the cache is empty
+            new = torch.empty if T else torch.zeros
+            out = new(Hq, self.head_dim, dtype=torch.float32, device=q.device)
         if T:
             rc = _lib.lib().ojasx_kv_decode_paged_device(
                 _vp(q), _vp(self.k_codes), _vp(self.k_scales), _vp(self.v_codes),
