@@ -139,6 +139,16 @@ def check(rc, what):
     return rc
 
 
+def raw_stream(device):
+    """The current stream of CUDA device index ``device`` as an integer, without
+    building a Stream object (1 to 2 us of a small call)."""
+    import torch
+    try:
+        return torch._C._cuda_getCurrentRawStream(device)
+    except AttributeError:
+        return torch.cuda.current_stream(device).cuda_stream
+
+
 def kernel_timing_enable(on=True):
     """Start (or stop) recording per-kernel start/stop events in the library;
     starting clears earlier records."""

@@ -24,7 +24,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from ._lib import DTYPE_BF16, DTYPE_F32, check, lib
+from ._lib import DTYPE_BF16, DTYPE_F32, check, lib, raw_stream
 
 
 def _dtype_tag(dt):
@@ -135,10 +135,20 @@ class SplitManifoldLUTLinear(nn.Module):
 
     # -- native handle --------------------------------------------------------
     def _key(self):
-        ts = [self.codebook, self.codes, self.scales, self.outlier_indices, self.outlier_values]
-        if self.bias is not None:
-            ts.append(self.bias)
-        return tuple((t.data_ptr(), t._version, t.device) for t in ts) + (self.num_outliers,)
+        # straight from the module's dicts: attribute access on a Module searches
+        # them by exceptions, a large part of a small call's host time
+        b, p = self._buffers, self._parameters
+        try:
+            ts = (b["codebook"], b["codes"], b["scales"], b["outlier_indices"],
+                  b["outlier_values"], p["bias"])
+        except KeyError:                 # a tensor registered as something else
+            ts = (self.codebook, self.codes, self.scales, self.outlier_indices,
+                  self.outlier_values, self.bias)
+        key = [self.num_outliers]
+        for t in ts:
+            if t is not None:
+                key += (t.data_ptr(), t._version, t.get_device())
+        return key
 
     def _handle(self):
         key = self._key()
@@ -218,14 +228,21 @@ class SplitManifoldLUTLinear(nn.Module):
         *bd, k = x.shape
         if k != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {k}")
-        xf = x.reshape(-1, k).contiguous()
-        y = torch.empty(xf.shape[0], self.out_features, device=x.device, dtype=x.dtype)
-        with torch.cuda.device(x.device):
-            h = self._handle()
-            check(lib().ojasx_linear_forward_device(
-                h, ctypes.c_void_p(xf.data_ptr()), ctypes.c_void_p(y.data_ptr()), xf.shape[0],
-                _dtype_tag(x.dtype), _stream_ptr(x.device)), "ojasx_linear_forward_device")
-        return y.view(*bd, self.out_features)
+        xf = x.contiguous()
+        y = torch.empty((*bd, self.out_features), device=x.device, dtype=x.dtype)
+        n = xf.numel() // k
+        device = x.get_device()
+        if device == torch.cuda.current_device():
+            self._launch(xf, y, n, device)
+        else:
+            with torch.cuda.device(device):
+                self._launch(xf, y, n, device)
+        return y
+
+    def _launch(self, xf, y, n, device):
+        rc = lib().ojasx_linear_forward_device(self._handle(), xf.data_ptr(), y.data_ptr(), n,
+                                               _dtype_tag(xf.dtype), raw_stream(device))
+        check(rc, "ojasx_linear_forward_device")
 
     def dequantize_weights(self) -> torch.Tensor:
         """Diagnostic dense weight (split_manifold_engine.py:252-267)."""

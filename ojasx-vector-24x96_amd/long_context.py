@@ -45,12 +45,11 @@ def _torch():
 
 
 def _vp(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _stream():
-    torch = _torch()
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _lib.raw_stream(_torch().cuda.current_device())
 
 
 def _require_gpu(t, what):
@@ -455,6 +454,8 @@ class PageTable:
         self.max_pages = max_pages
         self.sink_pages = sink_pages
         self.pages: List[int] = []
+        self.opened = 0                  # pages opened so far: changes whenever ``pages`` does
+        self.ids = np.zeros(max_pages, np.int32)   # ``pages`` as an array
         self._gen: List[int] = []
         self._next_gen = 0
         self.tail = 0
@@ -468,13 +469,21 @@ class PageTable:
         if len(self.pages) == self.max_pages:
             self._free.append(self.pages.pop(self.sink_pages))
             self._gen.pop(self.sink_pages)
+            self.ids[self.sink_pages:-1] = self.ids[self.sink_pages + 1:]
         self.pages.append(self._free.pop())
+        self.ids[len(self.pages) - 1] = self.pages[-1]
+        self.opened += 1
         self._gen.append(self._next_gen)
         self._next_gen += 1
         self.tail = 0
 
     def plan(self, n: int) -> np.ndarray:
         P = self.page_size
+        if n == 1:                       # a decode step: no page evicted within the call
+            if not self.pages or self.tail == P:
+                self._open_page()
+            self.tail += 1
+            return np.array([self.pages[-1] * P + self.tail - 1], np.int32)
         slots = np.empty(n, np.int32)
         gens = np.empty(n, np.int64)
         t = 0
@@ -538,7 +547,7 @@ class PagedCodeKVCache:
         self.k_scales = torch.zeros(shape, dtype=torch.float32, device=self.device)
         self.v_scales = torch.zeros_like(self.k_scales)
         self._bt = torch.zeros(max_resident_pages, dtype=torch.int32, device=self.device)
-        self._bt_pages: Optional[List[int]] = None
+        self._bt_opened = 0              # table.opened when _bt was written
 
     def _codebook(self, cb):
         torch = _torch()
@@ -587,11 +596,11 @@ class PagedCodeKVCache:
     def block_table(self):
         """Device int32 block table of the resident pages, in logical order."""
         torch = _torch()
-        pages = self.table.pages
-        if self._bt_pages != pages:
-            if pages:
-                self._bt[:len(pages)].copy_(torch.tensor(pages, dtype=torch.int32))
-            self._bt_pages = list(pages)
+        table = self.table
+        if self._bt_opened != table.opened:
+            n = len(table.pages)
+            self._bt[:n].copy_(torch.from_numpy(table.ids[:n]))
+            self._bt_opened = table.opened
         return self._bt
 
     def decode(self, q, scale_factor: float = -1.0, out=None):
