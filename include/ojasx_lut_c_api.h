@@ -113,10 +113,12 @@ OJASX_API void ojasx_destroy_linear(OjasxLinearHandle handle);
  * x 16-byte aligned) x . W^T on MFMA with W decoded from the codes.  Prefill
  * batches (from about 65 tokens, by shape and type; x 16-byte aligned) run on
  * larger tiles with scratch of the calling thread and stream, at most 256 MB
- * each and freed when the thread ends, and keep the handle's outliers once more
- * in groups of four entries of a row (9 bytes per entry and 9 to 36 per row),
- * made by the first such call; a call that is being captured, or finds no
- * memory, runs the kernel that needs neither. */
+ * each and freed when the thread ends (destroy a stream only when its calls
+ * are done: a new stream may get its handle, and with it the scratch), and
+ * keep the handle's outliers once more in groups of four entries of a row (9
+ * bytes per entry and 9 to 36 per row), made by the first such call; a call
+ * that is being captured, or finds no memory, runs the kernel that needs
+ * neither. */
 OJASX_API int ojasx_linear_forward_device(OjasxLinearHandle handle, const void *x, void *y,
                                           int batch_size, int dtype, void *stream);
 /* Many independent linears in one launch (no reference counterpart; the

@@ -230,6 +230,15 @@ constexpr int kScratchStreams = 4;
 int stream_scratch(hipStream_t st, size_t n, void **out);
 // Whether st can take calls that may allocate: not while it is being captured.
 bool may_allocate(hipStream_t st);
+// While one lives, this thread's calls on a stream that is not captured may
+// allocate although another stream is being captured (a capture in the default
+// mode makes every thread's allocations fail, and itself with them).
+struct AllocateWhileCapturing {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok;
+    AllocateWhileCapturing();
+    ~AllocateWhileCapturing();
+};
 // One linear handle's forward of B tokens (dtype F32 or BF16) on st.
 int linear_forward(void *h, const void *x, void *y, int B, int dtype, hipStream_t st);
 int linear_forward_fused(void *h, const float *x, float *y, int pro, const float *w, float eps,

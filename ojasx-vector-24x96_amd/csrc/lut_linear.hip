@@ -852,6 +852,7 @@ int forward(Linear *L, const void *x, void *y, int B, int dtype, hipStream_t st)
         g.M = L->M;
         g.Mp = L->Mp;
         if (reinterpret_cast<uintptr_t>(x) % 16 == 0 && gemm_pays(g, B, dtype) && may_allocate(st)) {
+            AllocateWhileCapturing relaxed;
             int rc = L->nnz ? outlier_groups(L, &g, st) : OJASX_OK;
             if (!rc) rc = launch_gemm(g, x, y, B, dtype, st);
             if (rc != OJASX_ERR_OOM) return rc;   // no memory: the kernel below needs none

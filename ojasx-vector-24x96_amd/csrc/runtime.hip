@@ -184,6 +184,14 @@ int stream_scratch(hipStream_t st, size_t n, void **out) {
     return OJASX_OK;
 }
 
+AllocateWhileCapturing::AllocateWhileCapturing() : ok(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+    if (!ok) (void)hipGetLastError();
+}
+
+AllocateWhileCapturing::~AllocateWhileCapturing() {
+    if (ok && hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
+}
+
 bool may_allocate(hipStream_t st) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &status) != hipSuccess) {

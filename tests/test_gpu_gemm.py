@@ -182,3 +182,30 @@ def test_capture_and_streams(pkg, dev):
     torch.cuda.synchronize()
     for a, b in zip(got, eager):
         assert torch.equal(a, b)
+
+
+def test_eager_call_beside_a_capture(pkg, dev):
+    """A handle's first prefill call (scratch and outlier groups to be allocated) on a stream of
+    its own while another stream is being captured: both give the results they give alone."""
+    import torch
+    M, K, B = 6912, 512, 260
+    d = make(M, K, B, 13, cb_bf16=True, x_bf16=True)
+    nat, alone = handle(pkg, d, M, K), handle(pkg, d, M, K)
+    x = torch.from_numpy(d["x"]).to(dev).bfloat16()
+    y = torch.empty(B, M, device=dev, dtype=torch.bfloat16)
+    want = forward(pkg, alone, x)
+    side, g, a = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.zeros(64, device=dev)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        a.add_(1)
+        rc = pkg.lib().ojasx_linear_forward_device(
+            nat.handle, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), B, 1,
+            ctypes.c_void_p(side.cuda_stream))
+        a.add_(1)
+    assert rc == 0, pkg.lib().ojasx_get_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert (a == 2 * (i + 1)).all()
