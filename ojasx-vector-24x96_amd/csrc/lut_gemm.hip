@@ -36,13 +36,14 @@
 #include <type_traits>
 
 #include "common.h"
+#include "lut_gemm_x.h"
 
 namespace ojx {
 
 namespace {
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 enum { kBf1 = 1, kHalf2 = 2, kHalf3 = 3 };
-constexpr int kGK = 64;             // input dims per step: four groups
+constexpr int kGK = kGemmStep;      // input dims per step: four groups
 constexpr long kGemmCUs = 256;
 constexpr size_t kGemmScratch = size_t(256) << 20;   // scratch bytes per pass over tokens
 
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
     constexpr int CB = 256 * 32;                     // bytes of a codebook piece
     constexpr int OT = BT >= 128 ? BT / 64 : 2;      // tokens per lane of an outlier read
     typedef typename std::conditional<PROD == kBf1, bf16x8_t, f16x8_t>::type frag_t;
-    static_assert(BT % 64 == 0 && (BT * 8) % NT == 0, "tile shapes");
+    static_assert(BT % 64 == 0 && (BT * 8) % NT == 0 && NT % 8 == 0, "tile shapes");
     extern __shared__ __align__(16) unsigned char sm[];
     unsigned char *cbs = sm;                         // [piece][half][256][16 bytes]
     unsigned char *xs = sm + PC * CB;                // [2 buffers][PX][BT][128 bytes]
@@ -111,28 +112,24 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
     constexpr int ROWB = PROD == kBf1 ? 0 : 1;       // planes are padded, bf16 x is not
     const unsigned char *xb = static_cast<const unsigned char *>(p.x);
     size_t xoff[XU];
-    int xst[XU], xk[XU];
+    int xst[XU];
     const size_t pitch = (size_t)(ROWB ? p.Kp : p.K) * 2;
+    const int xc = tid & 7;                          // NT % 8 == 0: the same for each of its units
 #pragma unroll
     for (int i = 0; i < XU; ++i) {
-        const int u = tid + i * NT, t = u >> 3, c = u & 7;
-        xoff[i] = (size_t)min(b0 + t, p.B - 1) * pitch + c * 16;
-        xst[i] = t * 128 + ((c ^ ((t >> 1) & 7)) << 4);
-        xk[i] = 8 * c;
+        const int t = (tid + i * NT) >> 3;
+        xoff[i] = (size_t)min(b0 + t, p.B - 1) * pitch;
+        xst[i] = t * 128 + ((xc ^ ((t >> 1) & 7)) << 4);
     }
     const size_t plane = (size_t)p.Bp * p.Kp * 2;
     uint4 xr[PXD][PX][XU];
     auto load_x = [&](int s, uint4 (&xr)[PX][XU]) __attribute__((always_inline)) {
+        const size_t o = gemm_x_unit(s, xc, ROWB ? p.Kp : p.K);
 #pragma unroll
         for (int q = 0; q < PX; ++q)
 #pragma unroll
-            for (int i = 0; i < XU; ++i) {
-                // bf16 x has no padding past K: the last step's units past it
-                // read the row's first unit and are zeroed when stored
-                const size_t o = ROWB ? (size_t)s * (kGK * 2)
-                                      : (s * kGK + xk[i] < p.K ? (size_t)s * (kGK * 2) : 0);
+            for (int i = 0; i < XU; ++i)
                 xr[q][i] = gld(reinterpret_cast<const uint4 *>(xb + q * plane + xoff[i] + o));
-            }
     };
     auto store_x = [&](int s, uint4 (&xr)[PX][XU]) __attribute__((always_inline)) {
         unsigned char *dst = xs + (s & 1) * (PX * PB);
@@ -141,7 +138,7 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int i = 0; i < XU; ++i) {
                 uint4 v = xr[q][i];
-                if (!ROWB && s * kGK + xk[i] >= p.K) v = make_uint4(0, 0, 0, 0);
+                if (!ROWB && s * kGK + 8 * xc >= p.K) v = make_uint4(0, 0, 0, 0);
                 *reinterpret_cast<uint4 *>(dst + q * PB + xst[i]) = v;
             }
     };

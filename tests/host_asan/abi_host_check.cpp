@@ -19,6 +19,7 @@
 #include <string>
 #include <vector>
 
+#include "lut_gemm_x.h"
 #include "ojasx_lut_c_api.h"
 
 static int g_fail = 0;
@@ -67,6 +68,20 @@ static void check_validation() {
     ojasx_destroy_moe(nullptr);
     ojasx_destroy_kv_cache(nullptr);
     CHECK(ojasx_get_compressed_size(nullptr) == 0, "size of null");
+}
+
+// ---- lut_gemm_kernel's reads of x: inside the tensor, at the unit's own dims
+static void check_gemm_reads() {
+    for (int K : {16, 32, 48, 64, 80, 112, 128, 272, 2560}) {
+        const int B = 5, steps = (K + ojx::kGemmStep - 1) / ojx::kGemmStep;
+        for (int s = 0; s < steps; ++s)
+            for (int c = 0; c < ojx::kGemmStep / 8; ++c) {
+                const size_t at = ojx::gemm_x_unit(s, c, K), k = (size_t)s * ojx::kGemmStep + 8 * c;
+                CHECK((size_t)(B - 1) * K * 2 + at + 16 <= (size_t)B * K * 2, "K %d step %d unit %d: byte %zu",
+                      K, s, c, at);
+                CHECK(k >= (size_t)K || at == 2 * k, "K %d step %d unit %d: byte %zu", K, s, c, at);
+            }
+    }
 }
 
 // ---- one linear, host pointers --------------------------------------------
@@ -264,6 +279,7 @@ static void check_timing() {
 
 int main() {
     check_validation();
+    check_gemm_reads();
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess) ndev = 0;
     std::printf("devices %d\n", ndev);

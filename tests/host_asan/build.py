@@ -55,7 +55,7 @@ def build(verbose=True):
         objs = list(ex.map(_compile_hip, srcs))
     drv = os.path.join(OUT, "abi_host_check.o")
     _run(["g++", "-std=c++17", "-O1", "-g", *GXX_SAN, "-D__HIP_PLATFORM_AMD__",
-          "-I", os.path.join(ROCM, "include"), "-I", os.path.join(ROOT, "include"),
+          "-I", os.path.join(ROCM, "include"), "-I", os.path.join(ROOT, "include"), "-I", CSRC,
           "-c", os.path.join(HERE, "abi_host_check.cpp"), "-o", drv])
     _run(["g++", *GXX_SAN, drv, *objs, "-o", EXE + ".tmp",
           "-L", os.path.join(ROCM, "lib"), "-lamdhip64", "-Wl,-rpath," + os.path.join(ROCM, "lib"),
