@@ -36,6 +36,9 @@ int DevBuf::ensure(size_t n) {
     hipError_t e = hipMalloc(&ptr, n);
     if (e != hipSuccess) {
         ptr = nullptr;
+        // reported here: a caller that goes on without the memory must not meet
+        // it again in its next hipGetLastError
+        (void)hipGetLastError();
         return hip_fail(e, "hipMalloc");
     }
     bytes = n;

@@ -9,6 +9,7 @@
 // of the reference's formulas (ojasx_lut_cpu.cpp:92-184, 213-365) written
 // here, so a silent corruption also fails.  Any sanitizer report aborts with
 // a non-zero status; the last line is "HOST_CHECK_OK" on success.
+#include <dlfcn.h>
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -32,6 +33,28 @@ static int g_fail = 0;
             ++g_fail;                                      \
         }                                                  \
     } while (0)
+
+// The library's allocations come through here.  With g_no_memory they fail: on
+// a device because the runtime is asked for more than it has, without one (where
+// the runtime's own calls all fail) by a stand-in that leaves the error for
+// hipGetLastError as the runtime does.
+static int g_devices = 0;
+static bool g_no_memory = false;
+static hipError_t g_left = hipSuccess;
+extern "C" hipError_t hipMalloc(void **p, size_t n) {
+    typedef hipError_t (*fn_t)(void **, size_t);
+    static const fn_t real = reinterpret_cast<fn_t>(dlsym(RTLD_NEXT, "hipMalloc"));
+    if (!g_devices && g_no_memory) return g_left = hipErrorOutOfMemory;
+    return real(p, g_no_memory ? size_t(1) << 60 : n);
+}
+extern "C" hipError_t hipGetLastError() {
+    typedef hipError_t (*fn_t)();
+    static const fn_t real = reinterpret_cast<fn_t>(dlsym(RTLD_NEXT, "hipGetLastError"));
+    if (g_devices) return real();
+    const hipError_t e = g_left;
+    g_left = hipSuccess;
+    return e;
+}
 
 static double rel_err(const std::vector<float> &y, const std::vector<double> &ref) {
     double num = 0, den = 0;
@@ -82,6 +105,18 @@ static void check_gemm_reads() {
                 CHECK(k >= (size_t)K || at == 2 * k, "K %d step %d unit %d: byte %zu", K, s, c, at);
             }
     }
+}
+
+// A failed allocation is reported by the call that made it and leaves no error
+// behind for the thread's next one.
+static void check_failed_allocation() {
+    std::vector<float> cb(256 * 16, 0.5f), sc(4, 1.f);
+    const uint8_t codes[8] = {0};
+    g_no_memory = true;
+    CHECK(!ojasx_create_linear(32, 4, 16, 256, cb.data(), codes, sc.data(), nullptr), "no memory");
+    g_no_memory = false;
+    const hipError_t e = hipGetLastError();
+    CHECK(e == hipSuccess, "left behind: %s", hipGetErrorString(e));
 }
 
 // ---- one linear, host pointers --------------------------------------------
@@ -146,6 +181,60 @@ static void check_linear(int K, int M, int D, int B, unsigned seed) {
           "sizes");
     ojasx_destroy_linear(h);
     std::printf("linear K=%d M=%d D=%d B=%d rel %.2e\n", K, M, D, B, e);
+}
+
+// ---- a prefill batch of the device entry point with no memory for its outlier
+// groups (the handle's first such call) or its scratch (a larger batch): the
+// call succeeds on the kernel that needs neither
+static void check_prefill_without_memory() {
+    const int K = 256, M = 4200, G = K / 16, most = 600;
+    std::mt19937 r(11);
+    std::normal_distribution<float> nd(0.f, 1.f);
+    std::vector<float> cb(256 * 16), sc(M, 0.75f), x((size_t)most * K), val(M);
+    std::vector<uint8_t> codes((size_t)M * G);
+    std::vector<int> rp(M + 1), col(M);
+    for (auto &v : cb) v = 0.02f * nd(r);
+    for (auto &v : x) v = nd(r);
+    for (auto &c : codes) c = (uint8_t)(r() & 255);
+    for (int m = 0; m < M; ++m) {
+        rp[m + 1] = m + 1;
+        col[m] = (int)(r() % K);
+        val[m] = nd(r);
+    }
+    OjasxLinearHandle h = ojasx_create_linear(K, M, 16, 256, cb.data(), codes.data(), sc.data(), nullptr);
+    CHECK(h && ojasx_set_linear_outliers(h, M, rp.data(), col.data(), val.data()) == 0, "create: %s",
+          ojasx_get_last_error());
+    float *xd = nullptr, *yd = nullptr;
+    CHECK(hipMalloc(reinterpret_cast<void **>(&xd), x.size() * 4) == hipSuccess &&
+              hipMalloc(reinterpret_cast<void **>(&yd), (size_t)most * M * 4) == hipSuccess &&
+              hipMemcpy(xd, x.data(), x.size() * 4, hipMemcpyHostToDevice) == hipSuccess, "buffers");
+    if (!h || !xd || !yd) return;
+    // no memory for the groups; memory; no memory for a larger batch's scratch
+    const int tokens[3] = {300, 300, most};
+    for (int i = 0; i < 3; ++i) {
+        const int B = tokens[i];
+        CHECK(hipMemset(yd, 0xff, (size_t)B * M * 4) == hipSuccess, "clear");
+        g_no_memory = i != 1;
+        const int rc = ojasx_linear_forward_device(h, xd, yd, B, 0, nullptr);
+        g_no_memory = false;
+        CHECK(rc == 0, "prefill call %d: %d %s", i, rc, ojasx_get_last_error());
+        std::vector<float> y((size_t)B * M), got;
+        CHECK(hipMemcpy(y.data(), yd, y.size() * 4, hipMemcpyDeviceToHost) == hipSuccess, "result");
+        std::vector<double> ref;
+        for (int b = 0; b < B; b += 37)
+            for (int m = 0; m < M; ++m) {
+                double a = 0;
+                for (int k = 0; k < K; ++k)
+                    a += (double)x[(size_t)b * K + k] * cb[(size_t)codes[(size_t)m * G + k / 16] * 16 + k % 16];
+                ref.push_back(sc[m] * a + (double)val[m] * x[(size_t)b * K + col[m]]);
+                got.push_back(y[(size_t)b * M + m]);
+            }
+        const double e = rel_err(got, ref);
+        CHECK(e < 1e-5, "prefill call %d: rel err %.3g", i, e);
+        std::printf("prefill %d tokens, %s memory: rel %.2e\n", B, i == 1 ? "with" : "no", e);
+    }
+    CHECK(hipFree(xd) == hipSuccess && hipFree(yd) == hipSuccess, "free");
+    ojasx_destroy_linear(h);
 }
 
 // ---- MoE, one token per call, host pointers --------------------------------
@@ -278,16 +367,17 @@ static void check_timing() {
 }
 
 int main() {
+    if (hipGetDeviceCount(&g_devices) != hipSuccess) g_devices = 0;
+    std::printf("devices %d\n", g_devices);
     check_validation();
     check_gemm_reads();
-    int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess) ndev = 0;
-    std::printf("devices %d\n", ndev);
-    if (ndev > 0) {
+    check_failed_allocation();
+    if (g_devices > 0) {
         check_linear(64, 40, 16, 3, 1);
         check_linear(2560, 300, 16, 2, 2);
         check_linear(96, 33, 24, 2, 3);
         check_linear(128, 17, 64, 1, 4);
+        check_prefill_without_memory();
         check_moe(5);
         check_kv(6);
         check_timing();

@@ -59,7 +59,7 @@ def build(verbose=True):
           "-c", os.path.join(HERE, "abi_host_check.cpp"), "-o", drv])
     _run(["g++", *GXX_SAN, drv, *objs, "-o", EXE + ".tmp",
           "-L", os.path.join(ROCM, "lib"), "-lamdhip64", "-Wl,-rpath," + os.path.join(ROCM, "lib"),
-          "-lpthread"])
+          "-lpthread", "-ldl"])
     os.replace(EXE + ".tmp", EXE)
     if verbose:
         print(f"built {EXE}")

@@ -46,3 +46,4 @@ def test_host_check_on_gpu():
     assert r.returncode == 0 and "HOST_CHECK_OK" in r.stdout
     assert "devices 0" not in r.stdout
     assert r.stdout.count("linear K=") >= 6 and "moe rel" in r.stdout and "kv rel" in r.stdout
+    assert r.stdout.count("no memory") == 2
