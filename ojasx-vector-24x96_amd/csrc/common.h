@@ -195,9 +195,8 @@ int launch_mm(const MmParams &p, int dtype, hipStream_t st);
 // K <= 65535; scratch of the calling thread and stream, so not under capture.
 struct LinearGemm {
     const uint8_t *codes;   // [S][Mp][16]
-    const void *cb_bf16;    // the codebook in bf16, where that is exact, or null
-    const void *cb_half;    // its fp16 pieces, scaled by 2^-ec, or null (split_codebook_half)
-    int ec;
+    const void *cb3;        // the codebook's exact bf16 pieces (split_codebook_bf16x3)
+    const void *cb_bf16;    // the codebook in bf16 (codebook_bf16), where that is exact, or null
     const float *scales;    // [M]
     const float *bias;      // [M] or null
     // The outliers in groups of four entries of one row, or null: row m's groups
@@ -215,11 +214,7 @@ int launch_gemm(const LinearGemm &g, const void *x, void *y, int B, int dtype, h
 // the others sized for nnz / 4 + M + 4 groups.
 int launch_outlier_groups(const int *rowp, const int *col, const float *val, int M, int K, int *gptr,
                           int *ocol, float *oval, int *orow, hipStream_t st);
-constexpr size_t kCbHalf = 2 * 256 * 16, kCbBf16 = 256 * 16;   // values of the two below
-// A 256 x 16 fp32 codebook as fp16 h + l of C * 2^-ec (2^-24 of every value),
-// laid out [piece][half][centroid][8]; false where that is not so: a value is
-// not finite, or a centroid's largest value is below 2^-16 of the codebook's.
-bool split_codebook_half(const float *cb, uint16_t *out, int *ec);
+constexpr size_t kCbBf16 = 256 * 16;   // values of the next
 // The codebook in bf16 laid out [half][centroid][8]; false unless exact.
 bool codebook_bf16(const float *cb, uint16_t *out);
 // Device scratch of the calling thread for work on st, at least n bytes: calls

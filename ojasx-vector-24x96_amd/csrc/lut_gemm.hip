@@ -15,18 +15,15 @@
 // operand feeding at most two MFMAs, x split in every workgroup) is bound by
 // the LDS and the VALU from about 100 tokens on.
 //
-// Products per multiply-add (kProd):
+// Products per multiply-add, both sides as exact bf16 pieces (bf16 keeps fp32's
+// exponent, so a value of any size beside any other is held whole):
 //  * kBf1: bf16 x and a codebook whose values are bf16: one, exact.
-//  * kHalf2: bf16 x, fp32 codebook: x as fp16 (a power-of-two scale per token
-//    brings its largest value to 2^14 .. 2^15, so the 8 significant bits of every
-//    value within 2^-29 of the largest are exact), C = h + l in fp16: two.
-//  * kHalf3: fp32 x, x = h + l and C = h + l: three, the product of the two low
-//    parts left out (2^-24 of the term).  h + l leaves 2^-24 of the value.
-// The sums are fp32 in the accumulators.  Against the exact three-way bf16
-// split (six products) the half splits measure the same error against 64 bits:
-// the fp32 accumulation sets it, with half as many steps here.
+//  * kBf3: bf16 x, fp32 codebook C = c1 + c2 + c3: three, exact.
+//  * kBf6: fp32 x = x1 + x2 + x3: the six products x_i c_j with i + j <= 4, as
+//    lut_mm32_kernel's; the three left out are below 2^-22 of the term.
+// The sums are fp32 in the accumulators.
 //
-// The x planes (fp16, K padded to 64 with zeros) and, where the layer has
+// The pieces of fp32 x (K padded to 64 with zeros) and, where the layer has
 // outliers, x transposed are written by gemm_prep_kernel into scratch of the
 // calling thread and stream.  Outliers: after the K loop the waves take the
 // tile's rows in turn, a lane holding BT / 64 neighbouring tokens: an entry is
@@ -41,8 +38,7 @@
 namespace ojx {
 
 namespace {
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-enum { kBf1 = 1, kHalf2 = 2, kHalf3 = 3 };
+enum { kBf1 = 1, kBf3 = 3, kBf6 = 6 };
 constexpr int kGK = kGemmStep;      // input dims per step: four groups
 constexpr long kGemmCUs = 256;
 constexpr size_t kGemmScratch = size_t(256) << 20;   // scratch bytes per pass over tokens
@@ -58,15 +54,14 @@ __device__ __forceinline__ V uld(const V *p) {
 
 struct GemmParams {
     const uint8_t *codes;           // [S][Mp][16]
-    const void *cbh;                // fp16: [piece][half][256][8]; bf16: [half][256][8]
+    const void *cb;                 // kBf1: bf16 [half][256][8]; else the pieces (split_codebook_bf16x3)
     const float *scales, *bias;
     const int *gptr, *orow, *ocol;  // outlier groups (LinearGemm) or null
     const float *oval;
-    const void *x;                  // kBf1: [B][K] bf16; else planes [piece][Bp][Kp] fp16
-    const int *ex;                  // [B] exponent of a token's scale (kHalf*)
+    const void *x;                  // bf16 x: [B][K]; fp32 x: its pieces [3][Bp][Kp] in bf16
     const void *xt;                 // [K + 1][Bp] x transposed (outliers), row K zero
     void *y;                        // [B][M]
-    int K, Kp, M, Mp, B, Bp, ec;    // ec: exponent of the codebook's scale
+    int K, Kp, M, Mp, B, Bp;
     int nr, nt, n_tiles;            // row tiles, token tiles, their product
 };
 }  // namespace
@@ -76,12 +71,11 @@ template <typename T, int PROD, int WT, int WR, int NWT, int NWR, int PXD>
 __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(2))) void lut_gemm_kernel(GemmParams p) {
     constexpr int NW = NWT * NWR, NT = 64 * NW;
     constexpr int BT = 32 * WT * NWT, BR = 32 * WR * NWR;
-    constexpr int PX = PROD == kHalf3 ? 2 : 1, PC = PROD == kBf1 ? 1 : 2;
+    constexpr int PX = PROD == kBf6 ? 3 : 1, PC = PROD == kBf1 ? 1 : 3;
     constexpr int XU = BT * 8 / NT;                  // 16-byte units of a step's plane per thread
     constexpr int PB = BT * 128;                     // bytes of a step's plane
     constexpr int CB = 256 * 32;                     // bytes of a codebook piece
     constexpr int OT = BT >= 128 ? BT / 64 : 2;      // tokens per lane of an outlier read
-    typedef typename std::conditional<PROD == kBf1, bf16x8_t, f16x8_t>::type frag_t;
     static_assert(BT % 64 == 0 && (BT * 8) % NT == 0 && NT % 8 == 0, "tile shapes");
     extern __shared__ __align__(16) unsigned char sm[];
     unsigned char *cbs = sm;                         // [piece][half][256][16 bytes]
@@ -96,20 +90,21 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
     if (tile >= p.n_tiles || (int)(blockIdx.x >> 3) >= per) return;
     const int b0 = (tile / p.nr) * BT, m0 = (tile % p.nr) * BR;
 
-    // ---- codebook into LDS
+    // ---- codebook into LDS, [centroid][half][piece] to piece planes
     {
         constexpr int NU = PC * CB / 16;
-        const uint4 *src = static_cast<const uint4 *>(p.cbh);
+        const uint4 *src = static_cast<const uint4 *>(p.cb);
 #pragma unroll
         for (int i = 0; i < (NU + NT - 1) / NT; ++i) {
             const int u = min(tid + i * NT, NU - 1);
-            reinterpret_cast<uint4 *>(cbs)[u] = gld(src + u);
+            const int to = PC == 1 ? u : u % PC * 512 + u / PC % 2 * 256 + u / (2 * PC);
+            reinterpret_cast<uint4 *>(cbs)[to] = gld(src + u);
         }
     }
     // ---- x staging: unit i of a plane = (token i / 8, dims 8 (i % 8) ..) of
     // the step; a token's 8 units are swizzled by (token / 2) % 8, so the 16
     // tokens a fragment read covers per phase fall in all 16 four-bank groups
-    constexpr int ROWB = PROD == kBf1 ? 0 : 1;       // planes are padded, bf16 x is not
+    constexpr int ROWB = PROD == kBf6 ? 1 : 0;       // planes are padded, bf16 x is not
     const unsigned char *xb = static_cast<const unsigned char *>(p.x);
     size_t xoff[XU];
     int xst[XU];
@@ -179,49 +174,49 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
         if (s + 1 < steps) store_x(s + 1, xr[u]);
         load_x(min(s + 1 + PXD, steps - 1), xr[u]);
         const unsigned char *xa = ar + (s & 1) * (PX * PB);
-        // kHalf3: a step's products into fresh tiles, then added to the sums:
-        // one rounding of the running sum per step instead of twelve
+        // kBf6: a step's products into fresh tiles, then added to the sums:
+        // one rounding of the running sum per step instead of 24
         f32x16_t d[WT][WR];
 #pragma unroll
         for (int t = 0; t < WT; ++t)
 #pragma unroll
             for (int r = 0; r < WR; ++r) {
-                if constexpr (PROD == kHalf3) d[t][r] = f32x16_t{};
+                if constexpr (PROD == kBf6) d[t][r] = f32x16_t{};
                 else d[t][r] = acc[t][r];
             }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            frag_t a[PX][WT], b[PC][WR];
+            bf16x8_t a[PX][WT], b[PC][WR];
 #pragma unroll
             for (int r = 0; r < WR; ++r)
 #pragma unroll
                 for (int q = 0; q < PC; ++q)
-                    b[q][r] = *reinterpret_cast<const frag_t *>(
+                    b[q][r] = *reinterpret_cast<const bf16x8_t *>(
                         br + q * CB + ((cc[0][r] >> (8 * g)) & 0xffu) * 16);
 #pragma unroll
             for (int t = 0; t < WT; ++t)
 #pragma unroll
                 for (int q = 0; q < PX; ++q)
-                    a[q][t] = *reinterpret_cast<const frag_t *>(xa + q * PB + t * (32 * 128) + go[g]);
+                    a[q][t] = *reinterpret_cast<const bf16x8_t *>(xa + q * PB + t * (32 * 128) + go[g]);
+            // the products x piece i of codebook piece j, i + j < PC, smallest
+            // first; every tile before the next product, so that neighbouring
+            // MFMAs do not wait for each other
 #pragma unroll
-            for (int t = 0; t < WT; ++t)
+            for (int k = PC - 1; k >= 0; --k)
 #pragma unroll
-                for (int r = 0; r < WR; ++r) {
-                    if constexpr (PROD == kBf1) {
-                        d[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][t], b[0][r], d[t][r], 0, 0, 0);
-                    } else {
-                        if constexpr (PROD == kHalf3)
-                            d[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][t], b[0][r], d[t][r], 0, 0, 0);
-                        d[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][t], b[1][r], d[t][r], 0, 0, 0);
-                        d[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][t], b[0][r], d[t][r], 0, 0, 0);
-                    }
-                }
+                for (int i = 0; i <= (PX > 1 ? k : 0); ++i)
+#pragma unroll
+                    for (int t = 0; t < WT; ++t)
+#pragma unroll
+                        for (int r = 0; r < WR; ++r)
+                            d[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][t], b[k - i][r], d[t][r],
+                                                                              0, 0, 0);
         }
 #pragma unroll
         for (int t = 0; t < WT; ++t)
 #pragma unroll
             for (int r = 0; r < WR; ++r) {
-                if constexpr (PROD == kHalf3) acc[t][r] += d[t][r];
+                if constexpr (PROD == kBf6) acc[t][r] += d[t][r];
                 else acc[t][r] = d[t][r];
             }
 #pragma unroll
@@ -332,15 +327,10 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
                     const float4 f = *reinterpret_cast<const float4 *>(orow + tk);
                     o4[0] = f.x; o4[1] = f.y; o4[2] = f.z; o4[3] = f.w;
                 }
-                int4 ex = make_int4(0, 0, 0, 0);
-                if constexpr (PROD != kBf1) ex = *reinterpret_cast<const int4 *>(p.ex + b);
-                const int e4[4] = {ex.x, ex.y, ex.z, ex.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     if (!ok || b + j >= p.B) continue;
-                    float a = acc[t][r][4 * v4 + j];
-                    if constexpr (PROD != kBf1) a = ldexpf(a, e4[j] + p.ec);
-                    float yv = a * sc;
+                    float yv = acc[t][r][4 * v4 + j] * sc;
                     if (p.bias) yv += bs;
                     store_act(y, (size_t)(b + j) * p.M + m, yv + o4[j]);
                 }
@@ -348,34 +338,11 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-// Per token the biased exponent of its largest magnitude (one wave each): the
-// scale 2^(141 - e) brings that value to 2^14 .. 2^15; ex[b] = e - 141.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_scale_kernel(const T *x, int B, int K, int *ex) {
-    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (b >= B) return;
-    const T *row = x + (size_t)b * K;
-    uint32_t m = 0;
-    constexpr int U = 8;
-    for (int c = lane * 4; c < K; c += 256 * U) {
-        float4 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = load4_act(row, min(c + 256 * u, K - 4));
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            m = max(m, max(__float_as_uint(v[u].x) & 0x7fffffffu, __float_as_uint(v[u].y) & 0x7fffffffu));
-            m = max(m, max(__float_as_uint(v[u].z) & 0x7fffffffu, __float_as_uint(v[u].w) & 0x7fffffffu));
-        }
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
-    if (lane == 0) ex[b] = max((int)(m >> 23), 1) - 141;
-}
-
-// 64 tokens x 64 dims: the fp16 planes (zero from K to Kp) and x transposed.
+// 64 tokens x 64 dims: the pieces of fp32 x (PX 3; zero from K to Kp) and x
+// transposed.
 template <typename T, int PX, bool XT>
 __global__ __launch_bounds__(256) void gemm_prep_kernel(const T *x, int B, int K, int Kp, int Bp,
-                                                       const int *ex, uint16_t *planes, T *xt) {
+                                                       uint16_t *planes, T *xt) {
     __shared__ T ts[64][72];                         // [dim][token], XT only
     const int k0 = blockIdx.x * 64, b0 = blockIdx.y * 64, tid = threadIdx.x;
     // thread: tokens tid / 8 + 32 i, dims 8 (tid % 8) ..
@@ -393,17 +360,11 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const T *x, int B, int K
         for (int j = 0; j < 8; ++j) v[j] = in ? v[j] : 0.f;
         if constexpr (PX > 0) {
             if (b < B && k < Kp) {
-                const int e = -ex[b];
-                f16x8_t ph, pl;
+                bf16x8_t pc[3];
+                split3_trunc(v, pc);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float f = ldexpf(v[j], e);
-                    ph[j] = (_Float16)f;
-                    pl[j] = (_Float16)(f - (float)ph[j]);
-                }
-                uint16_t *d = planes + (size_t)b * Kp + k;
-                *reinterpret_cast<f16x8_t *>(d) = ph;
-                if constexpr (PX == 2) *reinterpret_cast<f16x8_t *>(d + (size_t)Bp * Kp) = pl;
+                for (int q = 0; q < PX; ++q)
+                    *reinterpret_cast<bf16x8_t *>(planes + ((size_t)q * Bp + b) * Kp + k) = pc[q];
             }
         }
         if constexpr (XT)
@@ -479,7 +440,7 @@ namespace {
 template <typename T, int PROD, int WT, int WR, int NWT, int NWR, int PXD>
 int launch_gemm_tile(GemmParams p, hipStream_t st) {
     constexpr int NT = 64 * NWT * NWR, BT = 32 * WT * NWT, BR = 32 * WR * NWR;
-    constexpr int PX = PROD == kHalf3 ? 2 : 1, PC = PROD == kBf1 ? 1 : 2;
+    constexpr int PX = PROD == kBf6 ? 3 : 1, PC = PROD == kBf1 ? 1 : 3;
     constexpr size_t stage = (size_t)PC * 8192 + 2 * PX * BT * 128;
     constexpr size_t sums = (size_t)NWR * 32 * (BT + 4) * sizeof(float);
     const size_t lds = p.gptr ? std::max(stage, sums) : stage;
@@ -496,47 +457,61 @@ int launch_gemm_tile(GemmParams p, hipStream_t st) {
 }
 
 // Tile by how full it leaves the 256 CUs (one workgroup's K loop is a fixed
-// time, whatever the batch).  Measured, 2560 -> 6912, us per call:
-//   tokens              512    1024   2048        (fp32: 512  1024  2048)
-//   64 tok x 128 rows   47.6   81.8   137.8               97   173   305
-//   128 x 128           50.3   72.9   132.9              100   149   286
-//   256 x 256          103.7  107.7   119.4         (spills as fp32)
+// time, whatever the batch).  Measured, us per call, tokens x rows of a tile:
+//   one product, 2560 -> 6912, tokens     512   1024   2048
+//     64 x 128                           47.6   81.8  137.8
+//     128 x 128                          50.3   72.9  132.9
+//     256 x 256                         103.7  107.7  119.4
 // 128 x 128 from 384 tiles (9728 -> 2560 at 1024 tokens, 160 tiles: 176 against
-// 143 us); 256 x 256 for bf16 x where its last round of workgroups is at least
-// four fifths full (2560 -> 19456 at 1024 tokens, 304 tiles: 209 against 160 us).
+// 143 us); 256 x 256 where its last round of workgroups is at least four fifths
+// full (2560 -> 19456 at 1024 tokens, 304 tiles: 209 against 160 us).
+//   six products (three), tokens          256        512        1024       2048
+//     64 x 128                          73 (46)   130 (72)   240 (132)  429 (229)
+//     128 x 128                        101 (60)   115 (63)   225 (110)  448 (215)
+//     128 x 256                        168 (91)   171 (96)   197 (106)  393 (193)
+// Their times go by whole rounds of workgroups over the CUs: six products 61 us
+// a round and 9, 112 and 195; three 31 and 13, 51 and 10, 93.  The least of the
+// three sums is also the fastest at 9728 -> 2560, 2560 -> 19456, 2560 -> 2560 and
+// 512 -> 4096.
 template <typename T, int PROD>
 int launch_gemm_prod(const GemmParams &p, hipStream_t st) {
-    const long mid = (long)((p.M + 127) / 128) * ((p.B + 127) / 128);
-    if constexpr (PROD != kHalf3) {
-        const long big = (long)((p.M + 255) / 256) * ((p.B + 255) / 256);
-        if (5 * big >= 4 * kGemmCUs * ((big + kGemmCUs - 1) / kGemmCUs))
+    auto tiles = [&](int rows, int tokens) {
+        return (long)((p.M + rows - 1) / rows) * ((p.B + tokens - 1) / tokens);
+    };
+    auto rounds = [&](int rows, int tokens) { return (tiles(rows, tokens) + kGemmCUs - 1) / kGemmCUs; };
+    if constexpr (PROD == kBf1) {
+        if (5 * tiles(256, 256) >= 4 * kGemmCUs * rounds(256, 256))
             return launch_gemm_tile<T, PROD, 4, 2, 2, 4, 1>(p, st);
+        if (2 * tiles(128, 128) >= 3 * kGemmCUs) return launch_gemm_tile<T, PROD, 2, 2, 2, 2, 2>(p, st);
+        return launch_gemm_tile<T, PROD, 1, 1, 2, 4, 2>(p, st);
+    } else {
+        constexpr bool six = PROD == kBf6;
+        const long small = (six ? 61 : 31) * rounds(128, 64) + (six ? 9 : 13);
+        const long mid = (six ? 112 : 51) * rounds(128, 128) + (six ? 0 : 10);
+        const long big = (six ? 195 : 93) * rounds(256, 128);
+        if (big <= mid && big <= small) {
+            if constexpr (six) return launch_gemm_tile<T, PROD, 4, 1, 1, 8, 1>(p, st);
+            else return launch_gemm_tile<T, PROD, 2, 2, 2, 4, 1>(p, st);
+        }
+        if (mid <= small) return launch_gemm_tile<T, PROD, 2, 1, 2, 4, 1>(p, st);
+        return launch_gemm_tile<T, PROD, 1, 1, 2, 4, six ? 2 : 1>(p, st);
     }
-    if (2 * mid >= 3 * kGemmCUs) return launch_gemm_tile<T, PROD, 2, 2, 2, 2, PROD == kHalf3 ? 1 : 2>(p, st);
-    return launch_gemm_tile<T, PROD, 1, 1, 2, 4, 2>(p, st);
 }
 
-template <typename T>
-int launch_prep(const GemmParams &p, const void *x, int *ex, void *planes, void *xt, int px, hipStream_t st) {
-    const T *xp = static_cast<const T *>(x);
+// The pieces of fp32 x (planes) and x transposed (xt), where they are wanted.
+int launch_prep(const GemmParams &p, const void *x, bool f32, void *planes, void *xt, hipStream_t st) {
     const dim3 grid(xt ? p.K / 64 + 1 : p.Kp / 64, (p.B + 63) / 64);   // x^T: rows 0 .. K
-    if (px) {
-        OJX_LAUNCH((gemm_scale_kernel<T>), dim3((p.B + 3) / 4), dim3(256), 0, st, xp, p.B, p.K, ex);
-        OJX_HIP(hipGetLastError());
-    }
     uint16_t *pl = static_cast<uint16_t *>(planes);
-    T *tt = static_cast<T *>(xt);
-    const int *cex = ex;
-    if (px == 2 && xt)
-        OJX_LAUNCH((gemm_prep_kernel<T, 2, true>), grid, dim3(256), 0, st, xp, p.B, p.K, p.Kp, p.Bp, cex, pl, tt);
-    else if (px == 2)
-        OJX_LAUNCH((gemm_prep_kernel<T, 2, false>), grid, dim3(256), 0, st, xp, p.B, p.K, p.Kp, p.Bp, cex, pl, tt);
-    else if (px == 1 && xt)
-        OJX_LAUNCH((gemm_prep_kernel<T, 1, true>), grid, dim3(256), 0, st, xp, p.B, p.K, p.Kp, p.Bp, cex, pl, tt);
-    else if (px == 1)
-        OJX_LAUNCH((gemm_prep_kernel<T, 1, false>), grid, dim3(256), 0, st, xp, p.B, p.K, p.Kp, p.Bp, cex, pl, tt);
+    if (!f32)
+        OJX_LAUNCH((gemm_prep_kernel<__hip_bfloat16, 0, true>), grid, dim3(256), 0, st,
+                   static_cast<const __hip_bfloat16 *>(x), p.B, p.K, p.Kp, p.Bp, pl,
+                   static_cast<__hip_bfloat16 *>(xt));
     else if (xt)
-        OJX_LAUNCH((gemm_prep_kernel<T, 0, true>), grid, dim3(256), 0, st, xp, p.B, p.K, p.Kp, p.Bp, cex, pl, tt);
+        OJX_LAUNCH((gemm_prep_kernel<float, 3, true>), grid, dim3(256), 0, st, static_cast<const float *>(x),
+                   p.B, p.K, p.Kp, p.Bp, pl, static_cast<float *>(xt));
+    else
+        OJX_LAUNCH((gemm_prep_kernel<float, 3, false>), grid, dim3(256), 0, st, static_cast<const float *>(x),
+                   p.B, p.K, p.Kp, p.Bp, pl, static_cast<float *>(xt));
     OJX_HIP(hipGetLastError());
     return OJASX_OK;
 }
@@ -545,14 +520,13 @@ int launch_prep(const GemmParams &p, const void *x, int *ex, void *planes, void 
 
 // Where the batched kernel's workgroups (32 rows x 64 tokens for bf16 x, 64 x 32
 // for fp32) no longer fit one per CU, each further round of them costs about
-// 21 us at 2560 inputs, and the tiles above start at 30 us (one product) or 52
-// (two and three, the x planes' two launches included): 2560 -> 6912 at 128
-// tokens 30.9 against 43.2 us in bf16; fp32 54 against 48 at 128 (two rounds),
-// 57.6 against 89 at 256 (four).  At 9728 inputs two rounds lose already (161
-// against 243 us for 2560 rows at 256 fp32 tokens).
+// 21 us at 2560 inputs, and the tiles above start at 30 us (one product), 43
+// (three) or 70 (six, the x planes' launch included): 2560 -> 6912 at 128 tokens
+// 30.9 against 43.2 us in bf16; fp32 70 against 50 at 128 (two rounds), 73
+// against 96 at 256 (four).  At 9728 inputs two rounds lose already (210 against
+// 246 us for 2560 rows at 256 fp32 tokens).
 bool gemm_pays(const LinearGemm &g, int B, int dtype) {
     const bool f32 = dtype == OJASX_DTYPE_F32;
-    if (!(g.cb_half || (!f32 && g.cb_bf16))) return false;
     const long wgs = f32 ? (long)((g.M + 63) / 64) * ((B + 31) / 32) : (long)((g.M + 31) / 32) * ((B + 63) / 64);
     const bool one = !f32 && g.cb_bf16;
     return B > 64 && wgs > (one || g.K >= 4096 ? kGemmCUs : 2 * kGemmCUs);
@@ -560,12 +534,12 @@ bool gemm_pays(const LinearGemm &g, int B, int dtype) {
 
 int launch_gemm(const LinearGemm &g, const void *x, void *y, int B, int dtype, hipStream_t st) {
     const bool f32 = dtype == OJASX_DTYPE_F32;
-    const int prod = f32 ? kHalf3 : g.cb_bf16 ? kBf1 : kHalf2;
-    const int px = prod == kHalf3 ? 2 : prod == kHalf2 ? 1 : 0;
+    const int prod = f32 ? kBf6 : g.cb_bf16 ? kBf1 : kBf3;
+    const int px = f32 ? 3 : 0;                      // planes of x
     const size_t es = f32 ? 4 : 2;
     GemmParams p{};
     p.codes = g.codes;
-    p.cbh = prod == kBf1 ? g.cb_bf16 : g.cb_half;
+    p.cb = prod == kBf1 ? g.cb_bf16 : g.cb3;
     p.scales = g.scales;
     p.bias = g.bias;
     p.gptr = g.gptr;
@@ -576,36 +550,29 @@ int launch_gemm(const LinearGemm &g, const void *x, void *y, int B, int dtype, h
     p.Kp = (int)round_up(g.K, kGK);
     p.M = g.M;
     p.Mp = g.Mp;
-    p.ec = g.ec;
     // tokens per pass: the scratch stays below kGemmScratch
-    const size_t per_token = (size_t)px * p.Kp * 2 + (g.gptr ? (size_t)(p.K + 1) * es : 0) + 4;
+    const size_t per_token = (size_t)px * p.Kp * 2 + (g.gptr ? (size_t)(p.K + 1) * es : 0) + 1;
     const int most = (int)std::max<size_t>(256, kGemmScratch / per_token / 256 * 256);
     for (int b = 0; b < B; b += most) {
         const int nb = std::min(most, B - b);
         p.B = nb;
         p.Bp = (int)round_up(nb, 256);
         const size_t planes = (size_t)px * p.Bp * p.Kp * 2, xt = g.gptr ? (size_t)p.Bp * (p.K + 1) * es : 0;
-        const size_t exb = px ? round_up((size_t)p.Bp * 4, 256) : 0;
         unsigned char *ws = nullptr;
-        if (planes + xt + exb) {
-            int rc = stream_scratch(st, planes + xt + exb, reinterpret_cast<void **>(&ws));
+        if (planes + xt) {
+            int rc = stream_scratch(st, planes + xt, reinterpret_cast<void **>(&ws));
             if (rc) return rc;
         }
         const unsigned char *xb = static_cast<const unsigned char *>(x) + (size_t)b * g.K * es;
-        int *ex = px ? reinterpret_cast<int *>(ws) : nullptr;
-        void *pl = px ? ws + exb : nullptr, *tt = g.gptr ? ws + exb + planes : nullptr;
-        int rc = OJASX_OK;
-        if (px || tt)
-            rc = f32 ? launch_prep<float>(p, xb, ex, pl, tt, px, st)
-                     : launch_prep<__hip_bfloat16>(p, xb, ex, pl, tt, px, st);
+        void *pl = px ? ws : nullptr, *tt = g.gptr ? ws + planes : nullptr;
+        int rc = px || tt ? launch_prep(p, xb, f32, pl, tt, st) : OJASX_OK;
         if (rc) return rc;
         p.x = px ? pl : xb;
-        p.ex = ex;
         p.xt = tt;
         p.y = static_cast<unsigned char *>(y) + (size_t)b * g.M * es;
-        rc = prod == kHalf3 ? launch_gemm_prod<float, kHalf3>(p, st)
-             : prod == kHalf2 ? launch_gemm_prod<__hip_bfloat16, kHalf2>(p, st)
-                              : launch_gemm_prod<__hip_bfloat16, kBf1>(p, st);
+        rc = prod == kBf6 ? launch_gemm_prod<float, kBf6>(p, st)
+             : prod == kBf3 ? launch_gemm_prod<__hip_bfloat16, kBf3>(p, st)
+                            : launch_gemm_prod<__hip_bfloat16, kBf1>(p, st);
         if (rc) return rc;
     }
     return OJASX_OK;

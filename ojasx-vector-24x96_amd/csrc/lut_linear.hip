@@ -589,8 +589,7 @@ struct Linear {
     int K = 0, M = 0, D = 0, Kcb = 0, G = 0, S = 0, Mp = 0;
     bool has_bias = false;
     size_t nnz = 0;
-    int ec = 0;                // exponent of cb_half's scale
-    bool half = false, bf16 = false;   // which prefill codebooks follow cb3's pieces
+    bool bf16 = false;         // the codebook in bf16 (exact) follows cb3's pieces
     // The outliers in groups of four (LinearGemm): made by the first prefill call
     std::mutex group_lock;
     bool grouped = false;
@@ -842,10 +841,8 @@ int forward(Linear *L, const void *x, void *y, int B, int dtype, hipStream_t st)
         (dtype != OJASX_DTYPE_F32 || reinterpret_cast<uintptr_t>(x) % 16 == 0)) {
         LinearGemm g{};
         g.codes = L->codes.as<uint8_t>();
-        const uint16_t *pieces = L->cb3.as<uint16_t>() + kCb3Bytes / 2;
-        g.cb_half = L->half ? pieces : nullptr;
-        g.cb_bf16 = L->bf16 ? pieces + kCbHalf : nullptr;
-        g.ec = L->ec;
+        g.cb3 = L->cb3.ptr;
+        g.cb_bf16 = L->bf16 ? L->cb3.as<uint16_t>() + kCb3Bytes / 2 : nullptr;
         g.scales = L->scales.as<float>();
         g.bias = L->has_bias ? L->bias.as<float>() : nullptr;
         g.K = L->K;
@@ -1050,11 +1047,10 @@ OJASX_API OjasxLinearHandle ojasx_create_linear(int in_features, int out_feature
     }
     if (!rc) rc = upload(L->codebook, cb.data(), cb.size() * sizeof(float));
     if (!rc && L->D == 16) {   // the grouped kernel's MFMA operand
-        // the three pieces, then the prefill kernel's operands: fp16 halves, bf16
-        std::vector<uint16_t> cb3(kCb3Bytes / 2 + kCbHalf + kCbBf16);
+        // the three pieces, then the codebook in bf16
+        std::vector<uint16_t> cb3(kCb3Bytes / 2 + kCbBf16);
         split_codebook_bf16x3(cb.data(), cb3.data());
-        L->half = split_codebook_half(cb.data(), cb3.data() + kCb3Bytes / 2, &L->ec);
-        L->bf16 = codebook_bf16(cb.data(), cb3.data() + kCb3Bytes / 2 + kCbHalf);
+        L->bf16 = codebook_bf16(cb.data(), cb3.data() + kCb3Bytes / 2);
         rc = upload(L->cb3, cb3.data(), cb3.size() * 2);
     }
     if (!rc) rc = upload(L->scales, sc.data(), sc.size() * sizeof(float));

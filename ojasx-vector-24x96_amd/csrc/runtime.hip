@@ -4,7 +4,6 @@
 // ojasx_lut_c_api.cpp:17-31 (version and backend strings); the strings name
 // this engine instead of the reference's CPU backends.
 #include <algorithm>
-#include <cmath>
 #include <cstdarg>
 #include <cstring>
 #include <map>
@@ -89,52 +88,6 @@ void split_codebook_bf16x3(const float *cb, uint16_t *out) {
                 o[8] = h2;
                 o[16] = h3;
             }
-}
-
-namespace {
-// v (|v| <= 2^15) in fp16, rounded to nearest even; *back its value
-uint16_t half_rne(float v, float *back) {
-    uint32_t u;
-    memcpy(&u, &v, 4);
-    const uint32_t sign = u & 0x80000000u;
-    u ^= sign;
-    if (u < 0x38800000u) {                         // below 2^-14: multiples of 2^-24
-        float a;
-        memcpy(&a, &u, 4);
-        a = (a + 0.5f) - 0.5f;                     // 0.5's last place is 2^-24
-        *back = sign ? -a : a;
-        return (uint16_t)(sign >> 16 | (uint32_t)(a * 16777216.f));
-    }
-    u += 0xfffu + ((u >> 13) & 1u);
-    u &= ~0x1fffu;
-    const uint32_t b = u | sign;
-    memcpy(back, &b, 4);
-    return (uint16_t)(sign >> 16 | (u - 0x38000000u) >> 13);
-}
-}  // namespace
-
-bool split_codebook_half(const float *cb, uint16_t *out, int *ec) {
-    float mx = 0.f, cm[256] = {};
-    for (int i = 0; i < 256 * 16; ++i) {
-        if (!std::isfinite(cb[i])) return false;
-        cm[i / 16] = std::max(cm[i / 16], std::fabs(cb[i]));
-        mx = std::max(mx, cm[i / 16]);
-    }
-    for (float c : cm)
-        if (c > 0.f && (double)c < std::ldexp((double)mx, -16)) return false;
-    int e = 15;
-    if (mx > 0.f) (void)std::frexp(mx, &e);
-    *ec = e - 15;
-    const double scale = std::ldexp(1.0, -*ec);
-    for (int c = 0; c < 256; ++c)
-        for (int d = 0; d < 16; ++d) {
-            const float v = (float)(cb[c * 16 + d] * scale);   // exact
-            float h, l;
-            const size_t at = ((size_t)(d / 8) * 256 + c) * 8 + d % 8;
-            out[at] = half_rne(v, &h);
-            out[2 * 256 * 8 + at] = half_rne(v - h, &l);
-        }
-    return true;
 }
 
 bool codebook_bf16(const float *cb, uint16_t *out) {

@@ -55,7 +55,7 @@ def reference(d, rows=None):
     return no.linear_fp64(x, d["codebook"], d["codes"], d["scales"], d["bias"], d["csr"])
 
 
-# (rows, inputs, tokens): 64 x 128 tiles; 128 x 128; 256 x 256 where bf16 x takes it
+# (rows, inputs, tokens): every tile shape of each product kind among them
 SHAPES = [(6912, 256, 65), (6912, 2560, 130), (300, 208, 3300), (2049, 80, 1100), (129, 16, 8200),
           (1000, 80, 6200), (2049, 64, 5800), (6912, 272, 2000)]
 
@@ -63,7 +63,7 @@ SHAPES = [(6912, 256, 65), (6912, 2560, 130), (300, 208, 3300), (2049, 80, 1100)
 @pytest.mark.parametrize("M,K,B", SHAPES)
 @pytest.mark.parametrize("kind", ["bf16", "bf16_x", "fp32"])
 def test_prefill_shapes(pkg, dev, M, K, B, kind):
-    """One product (bf16 x and codebook), two (bf16 x, fp32 codebook), three (fp32 x)."""
+    """One product (bf16 x and codebook), three (bf16 x, fp32 codebook), six (fp32 x)."""
     import torch
     d = make(M, K, B, M + K + B, cb_bf16=kind == "bf16", x_bf16=kind != "fp32")
     nat = handle(pkg, d, M, K)
@@ -126,10 +126,9 @@ def test_outlier_groups(pkg, dev, kind):
 
 
 def test_scales_of_tokens_and_codebook(pkg, dev):
-    """Tokens of very different size (each has its own scale), all-zero tokens, one value 10^4
-    times the others; a codebook of tiny values, and one whose unused centroid is 10^9 times the
-    used ones (too wide for its half pieces: the batched kernel).  Error per token, relative to
-    the token's largest output."""
+    """Tokens of very different size, all-zero tokens, one value 10^4 times the others; a codebook
+    of tiny values, and one whose unused centroid is 10^9 times the used ones.  Error per token,
+    relative to the token's largest output."""
     import torch
     M, K, B = 6912, 512, 260
     d = make(M, K, B, 9)
@@ -150,6 +149,79 @@ def test_scales_of_tokens_and_codebook(pkg, dev):
         top = np.abs(want).max(1, keepdims=True)
         assert not y[7].any()
         assert (np.abs(y - want) / np.where(top > 0, top, 1)).max() < 1e-5, case
+
+
+@pytest.mark.parametrize("bf16_x", [False, True])
+@pytest.mark.parametrize("wide", ["x", "codebook"])
+def test_wide_range_inside_a_token(pkg, dev, wide, bf16_x):
+    """One value of a token 1 to 3e38 times the others in a place where a third of the rows have
+    a zero centroid and a third a centroid that is zero in that dim alone; and a codebook whose
+    dims 8 .. 15 are 1 to 3e-30 times dims 0 .. 7, with x zero in dims 0 .. 7.  Both are products
+    of ordinary size for those rows, held as if the large values were not there: the error
+    against 64 bits, relative to the token's largest output over those rows, is that of fp32 sums
+    (3e-7; the exact pieces leave 2^-22 of a term and sums of 96 rounded terms), plus the output's
+    own rounding in bf16 (8 significant bits to nearest: 2^-8 of the value)."""
+    import torch
+    M, K, B, dim = 6912, 512, 320, 16 * 5 + 3
+    d = make(M, K, B, 21, density=0.0, x_bf16=bf16_x)
+    d["bias"], d["csr"] = None, None
+    d["codebook"][0] = 0
+    d["codebook"][1, dim % 16] = 0
+    d["codes"] = np.maximum(d["codes"], 2)
+    rows = np.arange(M) % 3 < 2                       # the rows that do not see the large values
+    if wide == "x":
+        d["codes"][::3, dim // 16], d["codes"][1::3, dim // 16] = 0, 1
+        ratio = [1, 1e6, 1e7, 1e8, 1e10, 1e12, 1e20, 3e38]
+        d["x"][:, dim] = [ratio[b % 8] for b in range(B)]
+        if bf16_x:
+            d["x"] = to_bf16(d["x"])
+    else:
+        d["x"].reshape(B, -1, 16)[:, :, :8] = 0
+        rows[:] = True
+    for ratio in [1] if wide == "x" else [1, 1e-6, 1e-8, 1e-12, 3e-30]:
+        e = dict(d, codebook=d["codebook"].copy())
+        e["codebook"][:, 8:] *= np.float32(ratio)
+        nat = handle(pkg, e, M, K)
+        x = torch.from_numpy(d["x"]).to(dev)
+        y = forward(pkg, nat, x.bfloat16() if bf16_x else x).float().cpu().numpy()[:, rows]
+        W = no.dequantize(e["codebook"], e["codes"], e["scales"])[rows]
+        want = d["x"].astype(np.float64) @ W.astype(np.float64).T
+        err = np.abs(y - want) - (2.0 ** -8 * np.abs(want) if bf16_x else 0)
+        assert (err.max(1) / np.abs(want).max(1)).max() <= 3e-7, ratio
+
+
+# tokens that take each of the tiles of three and of six products at 6912 rows
+@pytest.mark.parametrize("B", [200, 512, 1024])
+@pytest.mark.parametrize("case", ["bf16_second", "bf16_third", "both_nine_bits", "codebook_17_bits",
+                                  "x_17_bits"])
+def test_every_product_counts(pkg, dev, B, case):
+    """Integers that need two or three bf16 pieces, in sums that are exact in fp32: a product left
+    out or a piece read from the wrong place changes the result.  bf16 x: a pair of inputs 1 and
+    -1 over centroids whose first piece is the same (and the second, for the third), so the
+    result is a difference of the lower pieces, which bf16 holds.  fp32 x: four inputs per token,
+    both sides of 9 to 11 bits, or one side of 17 bits and the other of at most 5."""
+    import torch
+    M, K = 6912, 256
+    r = np.random.default_rng(B)
+    i = np.arange(256)
+    value = {"bf16_second": (200 << 16) + 256 * (i % 128) + 37, "bf16_third": (200 << 16) + 256 * 90 + i % 120,
+             "both_nine_bits": 257 + 6 * i, "codebook_17_bits": 65793 + 257 * i, "x_17_bits": i % 31 + 1}[case]
+    d = dict(codebook=np.repeat(value[:, None], 16, 1).astype(np.float32), bias=None, csr=None,
+             codes=r.integers(0, 256, size=(M, K // 16)).astype(np.uint8), scales=np.ones(M, np.float32),
+             x=np.zeros((B, K), np.float32))
+    for b in range(B):
+        at = r.choice(K // 16, size=4, replace=False) * 16 + r.integers(0, 16, size=4)
+        if case.startswith("bf16"):
+            d["x"][b, at[:2]] = 1, -1
+        else:
+            top = {"both_nine_bits": (257, 1025), "codebook_17_bits": (1, 17), "x_17_bits": (65537, 1 << 17)}[case]
+            d["x"][b, at] = r.integers(*top, size=4) * r.choice([-1, 1], size=4)
+    nat = handle(pkg, d, M, K)
+    want = d["x"].astype(np.float64) @ no.dequantize(d["codebook"], d["codes"], d["scales"]).T
+    assert np.abs(want).max() < 2 ** 24
+    x = torch.from_numpy(d["x"]).to(dev)
+    y = forward(pkg, nat, x.bfloat16() if case.startswith("bf16") else x)
+    assert np.array_equal(y.float().cpu().numpy(), want)
 
 
 def test_capture_and_streams(pkg, dev):
