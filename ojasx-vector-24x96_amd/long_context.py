@@ -402,9 +402,11 @@ class OnlineSoftmaxBlockAttention:
         key, value, qp = self._pad_d(key), self._pad_d(value), self._pad_d(query)
         S_k = key.shape[2]
         # whole query blocks per pass: as many as keep the fp64 state (query,
-        # sums, maximum and weight of every row) within _STATE_BYTES
+        # sums, maximum and weight of every row) within _STATE_BYTES and the rows
+        # of a kv head within what an update takes (65535 blocks of 8)
         per_query = 8 * B * H_q * (2 * self._dpad + 2)
-        step = max(1, self._STATE_BYTES // (per_query * self.q_block_size)) * self.q_block_size
+        step = min(self._STATE_BYTES // per_query, 8 * 65535 // self.num_queries_per_kv)
+        step = max(1, step // self.q_block_size) * self.q_block_size
         outs = []
         for q_start in range(0, S_q, step):
             q_stop = min(q_start + step, S_q)

@@ -111,3 +111,19 @@ def test_strided_tensors_and_extremes(pkg, dev):
     out = att.forward(torch.zeros_like(q), k, v)
     bad = torch.isinf(out)
     assert bad[0, 4:8, :, 5].all() and int(bad.sum()) == 4 * S
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_more_rows_than_one_update_takes(pkg, dev, causal):
+    """600000 queries of one head of 16 dims: more than an update's 65535 blocks of 8 rows."""
+    import torch
+    S, T, D = 600000, 40, 16
+    g = torch.Generator().manual_seed(8)
+    q = torch.randn(1, 1, S, D, generator=g).to(dev)
+    k, v = (torch.randn(1, 1, T, D, generator=g).to(dev) for _ in range(2))
+    att = pkg.long_context.OnlineSoftmaxBlockAttention(1, 1, D, q_block_size=4096, causal=causal)
+    out = att.forward(q, k, v)
+    rows = [0, 1, T - 1, 4095, 4096, 524279, 524280, S - 1]
+    for r in rows:
+        ref = want(q[:, :, r:r + 1], k, v, causal, r)
+        assert np.abs(out[:, :, r:r + 1].cpu().numpy() - ref).max() <= 1e-6 * np.abs(ref).max(), r
