@@ -19,7 +19,10 @@
 //    fp64 (k_t converted exactly; q_r read at uniform addresses, so scalar
 //    operands), -inf where the causal mask hides the key (key position >
 //    query position, :133-139).  Chunk maximum m_c, p = exp(s - m_c) with
-//    p = 0 for -inf scores (the reference's guard, :144-156), l_c = sum p.
+//    p = 0 for -inf scores (the reference's guard, :144-156), l_c = sum p.  A
+//    chunk past the last position that a row of the block may see leaves an
+//    empty partial (m = -inf), and a float value row is added only to the rows
+//    that see its token, so a NaN or inf in a hidden one reaches no result.
 //    Values: thread (4 dims, token phase) accumulates p * vscale_t * v_t of
 //    every row over its tokens (int8 v: at head_dim 128 each thread's 32
 //    words loaded into registers at the start, otherwise the rows staged in
@@ -121,6 +124,15 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 }
 }  // namespace
 
+// The first and the last of the positions up to which rows r0 .. r0 + n - 1 of a
+// kv head (those below R) see the stream.
+__device__ __forceinline__ void horizons(const AttnParams &p, int r0, int n, long long *low, long long *top) {
+    const int rl = min(r0 + n, p.R) - 1;
+    const bool one = r0 / p.Sq == rl / p.Sq;          // rows of one query head
+    *low = p.causal ? p.qsp + (one ? r0 % p.Sq : 0) : 1LL << 62;
+    *top = p.causal ? p.qsp + (one ? rl % p.Sq : p.Sq - 1) : 1LL << 62;
+}
+
 template <int KT, int RB>
 __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
     typedef typename Elem<KT>::T T;
@@ -130,11 +142,19 @@ __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
     __shared__ double rm[4][RB], rl[4][RB];   // per-wave maxima and sums
     extern __shared__ uint4 vstage[];         // int8 tiles: the chunk's v rows [n][D] bytes
     const AttnWork wk = p.work[blockIdx.x];
-    const AttnTile tl = p.tiles[wk.tile];
     const int bh = blockIdx.y, b = bh / p.Hkv, h = bh - b * p.Hkv;
     const int r0 = blockIdx.z * RB;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int D = p.D, SW = 2 * D + 2;
+    const size_t slot0 = ((size_t)blockIdx.x * p.rows + (size_t)bh * p.R + r0) * (D + 2);
+    long long low, top;
+    horizons(p, r0, RB, &low, &top);
+    if (wk.pos > top) {
+        const int n = min(RB, p.R - r0) * (D + 2);
+        for (int i = tid; i < n; i += kANT) p.part[slot0 + i] = i % (D + 2) == D ? -INFINITY : 0.0;
+        return;
+    }
+    const AttnTile tl = p.tiles[wk.tile];
     const bool valid = tid < wk.n;
     const long long t = wk.t0 + min(tid, wk.n - 1);
     const T *kp = static_cast<const T *>(tl.k) + b * tl.sb + h * tl.sh + t * tl.st;
@@ -279,7 +299,10 @@ __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
     } else if (ts < TS) {
         const uint32_t *vs32 = reinterpret_cast<const uint32_t *>(vstage) + dq;
         const T *vp = vbase + 4 * dq;
-        for (int tt = ts; tt < wk.n; tt += TS) {
+        // float tiles: first the tokens that every row sees
+        const int all = kI8 ? wk.n : (int)max(0LL, min((long long)wk.n, low - wk.pos + 1));
+        int tt = ts;
+        for (; tt < all; tt += TS) {
             double v4[4];
             if constexpr (kI8) {
                 const uint32_t u = vs32[tt * NQ];
@@ -295,9 +318,25 @@ __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
                 for (int j = 0; j < 4; ++j) a4[r][j] = fma(wgt, v4[j], a4[r][j]);
             }
         }
+        if constexpr (!kI8) {
+            int see[RB];                              // row r sees the chunk's first see[r] tokens
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+                see[r] = (int)max(0LL, min((long long)wk.n, p.qsp + (r0 + r) % p.Sq - wk.pos + 1));
+            for (; tt < wk.n; tt += TS) {
+                double v4[4];
+                load_run<T, 4>(vp + tt * tl.st, v4);
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    const double wgt = pv[r][tt];
+                    if (tt < see[r])
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) a4[r][j] = fma(wgt, v4[j], a4[r][j]);
+                }
+            }
+        }
     }
     // the token phases summed in order, one row at a time through LDS
-    const size_t slot0 = ((size_t)blockIdx.x * p.rows + (size_t)bh * p.R + r0) * (D + 2);
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
 #pragma unroll
@@ -380,9 +419,8 @@ void attn_rows_kernel(AttnParams p, double *state, int n_work) {
     const bool rok = row < p.R;
     double *st = state + ((size_t)bh * p.R + min(row, p.R - 1)) * (2 * D + 2);
     const long long qpos = p.qsp + min(row, p.R - 1) % p.Sq;
-    // the last position any of the block's rows may see
-    const int rl = min(r0 + kRRows, p.R) - 1;
-    const long long top = p.causal ? p.qsp + (r0 / p.Sq == rl / p.Sq ? rl % p.Sq : p.Sq - 1) : 0x7fffffffffffffffLL;
+    long long low, top;
+    horizons(p, r0, kRRows, &low, &top);
 
     uint4 kr[NU], vr[NU];
     double scr = 0.0;

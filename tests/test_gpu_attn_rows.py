@@ -127,3 +127,31 @@ def test_more_rows_than_one_update_takes(pkg, dev, causal):
     for r in rows:
         ref = want(q[:, :, r:r + 1], k, v, causal, r)
         assert np.abs(out[:, :, r:r + 1].cpu().numpy() - ref).max() <= 1e-6 * np.abs(ref).max(), r
+
+
+# (query heads, kv heads, queries, tokens, start, head dim)
+HIDDEN = [(4, 4, 300, 300, 0, 32), (4, 2, 301, 301, 0, 96), (4, 4, 300, 500, 200, 256), (4, 1, 75, 75, 0, 64),
+          (2, 2, 7, 700, 500, 128)]
+
+
+@pytest.mark.parametrize("shape", HIDDEN)
+@pytest.mark.parametrize("dt", ["float64", "bfloat16"])
+def test_hidden_values_reach_no_result(pkg, dev, shape, dt):
+    """A NaN and an inf row of v change exactly the queries that see them: row blocks over two
+    heads, and tokens that all rows of a block see, some, or none."""
+    import torch
+    Hq, Hk, S, T, start, D = shape
+    g = torch.Generator().manual_seed(D + S)
+    dtype = getattr(torch, dt)
+    q = torch.randn(1, Hq, S, D, generator=g).to(dtype).to(dev)
+    k, v = (torch.randn(1, Hk, T, D, generator=g).to(dtype).to(dev) for _ in range(2))
+    att = pkg.long_context.OnlineSoftmaxBlockAttention(Hq, Hk, D, causal=True)
+    ref = want(q, k, v, True, start)
+    tol = {"float64": 1e-12, "bfloat16": 1e-2}[dt] * np.abs(ref).max()
+    assert np.abs(att.forward(q, k, v, query_start_pos=start).double().cpu().numpy() - ref).max() <= tol
+    first = S // 2 + 1                                # the first query that sees the NaN
+    v[:, :, start + first] = float("nan")
+    v[:, :, start + S - 1] = float("inf")
+    out = att.forward(q, k, v, query_start_pos=start).double().cpu().numpy()
+    assert np.abs(out[:, :, :first] - ref[:, :, :first]).max() <= tol
+    assert np.isnan(out[:, :, first:]).all()
