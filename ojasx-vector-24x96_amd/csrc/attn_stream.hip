@@ -376,6 +376,9 @@ __global__ __launch_bounds__(kANT) void attn_tile_kernel(AttnParams p) {
 //  * The online update is the reference's (:129-163) per 32 tokens; row bounds
 //    past R, tokens past the item and causally hidden ones score -inf, and a
 //    step whose first token no row may see ends the run.
+//  * A hidden token's weight is 0, and the MFMA adds 0 times its v: a wave whose
+//    sums are not finite folds its tokens once more, one at a time and into the
+//    rows that see them alone.
 // With one run the accumulators start from the state and go back to it; with
 // several (too few row blocks for the chip) each run leaves partials for
 // attn_merge_kernel.
@@ -494,14 +497,17 @@ void attn_rows_kernel(AttnParams p, double *state, int n_work) {
     for (int k = 0; k < D / 4; ++k) q[k] = st[4 * k + g];
     f64x4_t o[D / 16];
     double m = -INFINITY, l = 0.0;
+    auto start = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int d = 0; d < D / 16; ++d)
+        for (int d = 0; d < D / 16; ++d)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[d][r] = nz == 1 && wt == 0 ? st[D + 16 * d + 4 * r + g] : 0.0;
-    if (nz == 1 && wt == 0) {
-        m = st[2 * D];
-        l = g == 0 ? st[2 * D + 1] : 0.0;
-    }
+            for (int r = 0; r < 4; ++r) o[d][r] = nz == 1 && wt == 0 ? st[D + 16 * d + 4 * r + g] : 0.0;
+        if (nz == 1 && wt == 0) {
+            m = st[2 * D];
+            l = g == 0 ? st[2 * D + 1] : 0.0;
+        }
+    };
+    start();
 
     if (w0 < w1) {
         // the step being loaded: item wi, its tokens t0 ..
@@ -570,7 +576,7 @@ void attn_rows_kernel(AttnParams p, double *state, int n_work) {
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const double pr = isinf(s[r]) ? 0.0 : exp(s[r] - safe);
+                const double e = exp(s[r] - safe), pr = isinf(s[r]) ? 0.0 : e;   // no branch round exp
                 l += pr;
                 s[r] = pr * vs[r];
             }
@@ -585,6 +591,41 @@ void attn_rows_kernel(AttnParams p, double *state, int n_work) {
             pos = pos1;
             cur = more;
             more = more1;
+        }
+    }
+    if constexpr (!kI8) {
+        bool bad = false;
+#pragma unroll
+        for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bad |= !(fabs(o[d][r]) < INFINITY);
+        if (__any(bad)) {
+            m = -INFINITY;
+            l = 0.0;
+            start();
+            for (int i = w0; i < w1; ++i) {
+                const AttnWork wk = p.work[i];
+                const AttnTile tl = p.tiles[wk.tile];
+                for (int tt = 16 * wt; tt < wk.n && wk.pos + tt <= top; tt += (tt & 15) == 15 ? 17 : 1) {
+                    const long long at = b * tl.sb + h * tl.sh + (wk.t0 + tt) * tl.st + g;
+                    const T *kt = static_cast<const T *>(tl.k) + at, *vt = static_cast<const T *>(tl.v) + at;
+                    double s = 0.0;
+#pragma unroll
+                    for (int k = 0; k < D / 4; ++k) s = fma(to_d(kt[4 * k]), q[k], s);
+                    s += __shfl_xor(s, 16, 64);
+                    s += __shfl_xor(s, 32, 64);
+                    s *= p.scale;
+                    if (p.causal && wk.pos + tt > qpos) continue;
+                    const double mn = fmax(m, s), safe = isinf(mn) ? 0.0 : mn;
+                    const double f = isinf(m) ? 0.0 : exp(m - safe), pr = isinf(s) ? 0.0 : exp(s - safe);
+                    m = mn;
+                    l = l * f + (g == 0 ? pr : 0.0);
+#pragma unroll
+                    for (int d = 0; d < D / 16; ++d)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) o[d][r] = fma(pr, to_d(vt[16 * d + 4 * r]), o[d][r] * f);
+                }
+            }
         }
     }
     l += __shfl_xor(l, 16, 64);

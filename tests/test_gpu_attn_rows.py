@@ -131,7 +131,10 @@ def test_more_rows_than_one_update_takes(pkg, dev, causal):
 
 # (query heads, kv heads, queries, tokens, start, head dim)
 HIDDEN = [(4, 4, 300, 300, 0, 32), (4, 2, 301, 301, 0, 96), (4, 4, 300, 500, 200, 256), (4, 1, 75, 75, 0, 64),
-          (2, 2, 7, 700, 500, 128)]
+          (2, 2, 7, 700, 500, 128),
+          # attn_rows_kernel: one head per row block; two; every step seen in part by some
+          (16, 16, 300, 600, 300, 128), (32, 8, 70, 1111, 1041, 64), (32, 8, 130, 1500, 1370, 80),
+          (16, 4, 512, 2048, 1536, 128)]
 
 
 @pytest.mark.parametrize("shape", HIDDEN)
@@ -155,3 +158,15 @@ def test_hidden_values_reach_no_result(pkg, dev, shape, dt):
     out = att.forward(q, k, v, query_start_pos=start).double().cpu().numpy()
     assert np.abs(out[:, :, :first] - ref[:, :, :first]).max() <= tol
     assert np.isnan(out[:, :, first:]).all()
+
+
+def test_infinite_value_in_a_partial_step(pkg, dev):
+    """attn_rows_kernel: +inf in the last value row of a step that is not full stays inf."""
+    import torch
+    q, k = torch.zeros(1, 16, 64, 64, device=dev), torch.zeros(1, 4, 2050, 64, device=dev)
+    v = torch.ones(1, 4, 2050, 64, device=dev)
+    v[:, 2, -1, 5] = float("inf")
+    out = pkg.long_context.OnlineSoftmaxBlockAttention(16, 4, 64, causal=False).forward(q, k, v)
+    assert torch.isinf(out[:, 8:12, :, 5]).all()
+    out[:, 8:12, :, 5] = 1
+    assert (out - 1).abs().max() < 1e-6
