@@ -562,6 +562,10 @@ class PagedCodeKVCache:
         return cb.to(self.device).contiguous()
 
     def append(self, k, v) -> None:
+        """Encode the tokens of ``k`` and ``v`` [S, H_kv, D] (or [H_kv, D]) into the
+        slots that the page table opens for them.  The slots are planned on the
+        host, so a captured append would write the same ones on every replay:
+        it raises, and the cache stays as it is."""
         torch = _torch()
         _require_gpu(k, "PagedCodeKVCache.append")
         _require_gpu(v, "PagedCodeKVCache.append")
@@ -571,23 +575,28 @@ class PagedCodeKVCache:
         if k.dim() != 3 or tuple(k.shape[1:]) != want or k.shape != v.shape:
             raise ValueError(f"k and v must be [S, {want[0]}, {want[1]}] of one shape")
         n = k.shape[0]
-        self.total_tokens_seen += n
         if n == 0:
             return
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("PagedCodeKVCache.append plans its slots on the host and cannot be "
+                               "captured: capture ojasx_kv_encode_append_device with a device slot "
+                               "mapping")
+        self.total_tokens_seen += n
         slots = self.table.plan(n)
         if n <= 64:                      # the slots travel with the launch
-            fn, at = _lib.lib().ojasx_kv_encode_append_host_slots, slots.ctypes.data
+            name, at = "ojasx_kv_encode_append_host_slots", slots.ctypes.data
         else:
             slots = torch.from_numpy(slots).to(self.device)
-            fn, at = _lib.lib().ojasx_kv_encode_append_device, slots.data_ptr()
+            name, at = "ojasx_kv_encode_append_device", slots.data_ptr()
         k = k.to(torch.float32).contiguous()
         v = v.to(torch.float32).contiguous()
         cbk = None if self.scalar_codes else _vp(self.k_codebook)
         cbv = None if self.scalar_codes else _vp(self.v_codebook)
-        rc = fn(_vp(k), _vp(v), n, self.num_kv_heads, self.head_dim, self.block_dim, cbk, cbv,
-                at, self.page_size, self.max_resident_pages, _vp(self.k_codes),
-                _vp(self.k_scales), _vp(self.v_codes), _vp(self.v_scales), _stream())
-        _lib.check(rc, "ojasx_kv_encode_append")
+        rc = getattr(_lib.lib(), name)(
+            _vp(k), _vp(v), n, self.num_kv_heads, self.head_dim, self.block_dim, cbk, cbv,
+            at, self.page_size, self.max_resident_pages, _vp(self.k_codes),
+            _vp(self.k_scales), _vp(self.v_codes), _vp(self.v_scales), _stream())
+        _lib.check(rc, name)
 
     @property
     def seq_len(self) -> int:

@@ -63,6 +63,31 @@ def test_append_slots_in_the_launch(pkg, dev, n, codebook):
         assert torch.equal(before, b.k_codes)
 
 
+@pytest.mark.parametrize("n", [1, 64, 65])
+def test_append_refuses_capture(pkg, dev, n):
+    """A captured append would write the same slots on every replay: it raises before the page
+    table moves, and the capture and later appends go on."""
+    import torch
+    cache = pkg.long_context.PagedCodeKVCache(2, 64, 16, page_size=16, max_resident_pages=8,
+                                              sink_pages=1, device=dev)
+    x = torch.randn(n, 2, 64, device=dev)
+    cache.append(x[:1], x[:1])
+    codes, a = cache.k_codes.clone(), torch.zeros(4, device=dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        a.add_(1)
+        with pytest.raises(RuntimeError, match="captured"):
+            cache.append(x, x)
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert (a == i + 1).all()
+    assert cache.seq_len == cache.total_tokens_seen == 1 and torch.equal(cache.k_codes, codes)
+    cache.append(x, x)
+    assert cache.seq_len == cache.total_tokens_seen == 1 + n
+
+
 def test_host_slots_refuses_more_than_64(pkg, dev):
     import torch
     t = torch.zeros(65, 1, 16, device=dev)
