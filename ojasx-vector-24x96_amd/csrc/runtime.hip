@@ -111,6 +111,7 @@ struct StreamScratch {
     } slot[kScratchStreams];
     unsigned long calls = 0;
     ~StreamScratch() {
+        AllocateWhileCapturing relaxed;
         for (Slot &s : slot) s.buf.release();
     }
 };

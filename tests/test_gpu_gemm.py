@@ -281,3 +281,38 @@ def test_eager_call_beside_a_capture(pkg, dev):
         g.replay()
         torch.cuda.synchronize()
         assert (a == 2 * (i + 1)).all()
+
+
+def test_thread_ends_beside_a_capture(pkg, dev):
+    """A thread that made prefill calls ends, and frees its scratch, while another thread's stream
+    is being captured: the capture goes on."""
+    import threading
+    import torch
+    M, K, B = 6912, 512, 260
+    d = make(M, K, B, 14)
+    nat = handle(pkg, d, M, K)
+    x = torch.from_numpy(d["x"]).to(dev)
+    called, end, out = threading.Event(), threading.Event(), []
+
+    def work():
+        out.append(forward(pkg, nat, x))
+        torch.cuda.synchronize()
+        called.set()
+        end.wait(60)
+
+    t = threading.Thread(target=work)
+    t.start()
+    assert called.wait(60)
+    a, g = torch.zeros(64, device=dev), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        a.add_(1)
+        end.set()
+        t.join(60)
+        a.add_(1)
+    assert not t.is_alive()
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert (a == 2 * (i + 1)).all()
+    assert torch.equal(out[0], forward(pkg, nat, x))
