@@ -116,9 +116,9 @@ OJASX_API void ojasx_destroy_linear(OjasxLinearHandle handle);
  * each and freed when the thread ends (destroy a stream only when its calls
  * are done: a new stream may get its handle, and with it the scratch), and
  * keep the handle's outliers once more in groups of four entries of a row (9
- * bytes per entry and 9 to 36 per row), made by the first such call; a call
- * that is being captured, or finds no memory, runs the kernel that needs
- * neither. */
+ * bytes per entry and 9 to 36 per row), made by the first such call, which
+ * waits for them; a call that is being captured, or finds no memory, runs the
+ * kernel that needs neither. */
 OJASX_API int ojasx_linear_forward_device(OjasxLinearHandle handle, const void *x, void *y,
                                           int batch_size, int dtype, void *stream);
 /* Many independent linears in one launch (no reference counterpart; the

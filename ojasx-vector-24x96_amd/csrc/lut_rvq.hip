@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kNT) void lut_rvq_kernel(RvqParams p) {
 // What bounds it: LDS reads of random codebook rows and the MFMAs of a padded
 // token tile, behind one staging round trip.  The kernel above reads a codebook
 // row for 4 tokens and runs the dots on the VALU: 6912 x 2560, two 8-bit stages
-// of block 16, 32 tokens 383 us against 26 here (bf16 x 410 against 19), 128
+// of block 16, 32 tokens 383 us against 23 here (bf16 x 410 against 19), 128
 // tokens 1474 against 82; error against 64 bits 1.34e-7 (1.63e-7 above).
 namespace {
 constexpr int kRvqNT = 512, kRvqWaves = kRvqNT / 64;
