@@ -215,9 +215,9 @@ __global__ __launch_bounds__(64 * NWT * NWR) __attribute__((amdgpu_waves_per_eu(
         constexpr std::integral_constant<int, PC - 1> top{};
         constexpr std::integral_constant<int, 0> first{};
         if constexpr (PROD == kBf6) {
-            // the step's small products before its large ones, whose operands
-            // are read again: the large partial sums are rounded four times
-            // instead of twenty.  Error against 64 bits 1.09e-7 -> 9.3e-8 at 2560
+            // the step's small products before its large ones (the compiler
+            // holds these operands in registers over the step): the large
+            // partial sums are rounded four times instead of twenty.  Error against 64 bits 1.09e-7 -> 9.3e-8 at 2560
             // inputs, 1.74e-7 -> 1.61e-7 at 9728, 8.0e-8 -> 5.9e-8 at 512, for
             // 0 to 1 % of the time (4 % at 9728 -> 2560 and 256 tokens)
 #pragma unroll
